@@ -16,6 +16,13 @@
 
 namespace g4 {
 
+// One row-per-half-wave launch over a single weight matrix (linear.hip, k_linear):
+// the values of matmul_quant / matmul_q8 / matmul_q4k, bit for bit. format:
+// G4_WEIGHT_*; meta: the quantized formats' scales. Returns 1, launching
+// nothing, for the shapes and alignments that form does not take.
+int launch_matmul_rows(uint32_t format, const float* x, const void* w, const uint16_t* meta, float* y, uint32_t M,
+                       uint32_t N, hipStream_t st);
+
 template <typename T>
 __device__ __forceinline__ T ldg_nt(const void* p) {
     typedef const __attribute__((address_space(1))) T* gp;

@@ -148,6 +148,28 @@ int add_segment(const char* who, LinearArgs* a, uint32_t i, const void* w, const
     return G4_OK;
 }
 
+// The engine's one-matrix matmuls (lmhead.hip) as one segment of k_linear. The
+// rule is what the row form can take: rows of 4 to 16 whole 256-column blocks
+// (the half-wave's lanes then hold the shader's partials in registers) and the
+// 16-byte loads' alignment (8 and 4 bytes for q8 and q4k rows). Within it the
+// row form is the faster one at every row count measured (kernel us, one
+// workgroup per row / this): f16 [262144][1536] 491.7 / 126.2 (6.38 TB/s),
+// [2048][1536] 7.4 / 5.1, [256][1536] 4.5 / 3.8, [1536][4096] 7.5 / 5.2.
+int launch_matmul_rows(uint32_t format, const float* x, const void* w, const uint16_t* meta, float* y, uint32_t M,
+                       uint32_t N, hipStream_t st) {
+    if (N % 256 || N / 256 < (uint32_t)kLinearMinJ || N / 256 > (uint32_t)kLinearMaxJ || M > 0x7fffffffu) return 1;
+    const uintptr_t w_align = format == G4_WEIGHT_F16 ? 15 : format == G4_WEIGHT_Q8 ? 7 : 3;
+    if ((reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(w) & w_align)) return 1;
+    LinearArgs a{};
+    a.x = x;
+    a.n_segs = 1;
+    a.total_rows = M;
+    a.seg[0] = LinearSegDev{w, meta, y, M, 0};
+    if (format == G4_WEIGHT_Q8) return launch_linear_n<kQ8>(a, N, st);
+    if (format == G4_WEIGHT_Q4K) return launch_linear_n<kQ4K>(a, N, st);
+    return launch_linear_n<kF16>(a, N, st);
+}
+
 // attn.linearQKV with the producer-side prep of the attention block as its
 // epilogue (src/engine.ts:2045-2091: linearQKV, then perHeadRmsNormNoWeight
 // on v, fusedPerHeadNormRope on q and k, kvCacheStore), in one launch. The

@@ -316,6 +316,8 @@ static dim3 matmul_grid(uint32_t M) {
 int g4_matmul_quant_f16(const float* input, const uint16_t* weight, float* output, g4_matmul_params p, void* stream) {
     if (!input || !weight || !output) return fail(G4_EINVAL, "matmulQuant: NULL pointer");
     if (p.M == 0) return G4_OK;
+    const int rc = launch_matmul_rows(G4_WEIGHT_F16, input, weight, nullptr, output, p.M, p.N, as_stream(stream));
+    if (rc <= 0) return rc;
     G4_LAUNCH(k_matmul_quant_f16, matmul_grid(p.M), dim3(kWG), 0, as_stream(stream), input, weight, output, p);
     G4_CHECK_LAUNCH("matmulQuant");
     return G4_OK;
@@ -326,6 +328,8 @@ int g4_matmul_q8(const float* input, const int8_t* qweight, const uint16_t* qsca
     if (!input || !qweight || !qscale || !output) return fail(G4_EINVAL, "matmulQ8: NULL pointer");
     if (p.N % 32) return fail(G4_EINVAL, "matmulQ8: N %u is not a multiple of 32", p.N);
     if (p.M == 0) return G4_OK;
+    const int rc = launch_matmul_rows(G4_WEIGHT_Q8, input, qweight, qscale, output, p.M, p.N, as_stream(stream));
+    if (rc <= 0) return rc;
     G4_LAUNCH(k_matmul_q8, matmul_grid(p.M), dim3(kWG), 0, as_stream(stream), input, qweight, qscale, output,
                        p);
     G4_CHECK_LAUNCH("matmulQ8");
@@ -337,6 +341,8 @@ int g4_matmul_q4k(const float* input, const uint32_t* qweight, const uint16_t* q
     if (!input || !qweight || !qmeta || !output) return fail(G4_EINVAL, "matmulQ4K: NULL pointer");
     if (p.N % 256) return fail(G4_EINVAL, "matmulQ4K: N %u is not a multiple of 256", p.N);
     if (p.M == 0) return G4_OK;
+    const int rc = launch_matmul_rows(G4_WEIGHT_Q4K, input, qweight, qmeta, output, p.M, p.N, as_stream(stream));
+    if (rc <= 0) return rc;
     G4_LAUNCH(k_matmul_q4k, matmul_grid(p.M), dim3(kWG), 0, as_stream(stream), input, qweight, qmeta, output,
                        p);
     G4_CHECK_LAUNCH("matmulQ4K");
