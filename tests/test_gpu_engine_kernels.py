@@ -1,5 +1,5 @@
 """GPU parity of the engine's own dispatches where their fast forms begin and end: the matmuls'
-row form. Every form evaluates the reference's f32 operations in the reference's
+row form and argmax's batches. Every form evaluates the reference's f32 operations in the reference's
 order, so the bar is bit equality with the oracle, which also covers the general forms on the other side of each rule.
 """
 import numpy as np
@@ -8,6 +8,7 @@ import torch
 
 from conftest import announce
 from g4attn import ops
+from oracle import closed_form as cf
 from oracle import oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -52,3 +53,15 @@ def test_matmul_forms(dev, fmt, M, N, offset):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(bits(out)[:M], want.view(np.uint32))
     assert float(out[M]) == 7.0
+
+
+@pytest.mark.parametrize("size,offset", [(1, 0), (3, 1), (4095, 0), (32768, 0), (32769, 0), (40000, 1), (70001, 2)])
+def test_argmax_forms(dev, size, offset):
+    announce(f"argmax size={size} offset={offset}")
+    rng = np.random.default_rng(size)
+    x = rng.integers(-3, 9, size=size).astype(np.float32)  # many ties
+    x[rng.integers(0, size, size=size // 5)] = np.nan
+    res = torch.full((1,), -1, dtype=torch.int32, device=dev)
+    ops.argmax(up(x, dev, offset), res, size)
+    torch.cuda.synchronize()
+    assert int(res.item()) == orc.argmax(x) == cf.argmax_rule(x)
