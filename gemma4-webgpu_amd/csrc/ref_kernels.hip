@@ -8,6 +8,11 @@
 //   softmax                 shaders/softmax.wgsl:7-46
 //   attnOutput              shaders/attn_output.wgsl:7-23        (f16 cache)
 //
+// attnScore, softmax and attnOutput also have forms for the sizes the engine
+// dispatches (k_attn_score_tile, k_softmax_reg, k_attn_output_chain): the same
+// operations in the same order on every value, so the same bits, with the work
+// of one value spread differently over threads and memory.
+//
 // They are the per-kernel drop-in surface (the engine's capture points
 // postRopeQ/K and attnOut sit between them, src/engine.ts:2086-2095) and the
 // unfused comparison path for the fused kernels. Arithmetic: every f32
@@ -76,6 +81,114 @@ __global__ __launch_bounds__(kWG) void k_attn_score(const float* __restrict__ q,
     scores[score_idx] = dot * p.scale;
 }
 
+// x * y rounded once, x an f16 value widened exactly: v_fma_mix_f32 with an
+// addend of -0 (x y + -0 is x y, its sign of zero included), one instruction
+// where widening and multiplying take two. `neg_zero` comes from opaque_neg_zero,
+// which keeps the compiler from folding the addition away.
+__device__ __forceinline__ float opaque_neg_zero() {
+    float z = -0.0f;
+    asm volatile("" : "+v"(z));
+    return z;
+}
+__device__ __forceinline__ float mul_f16(f16 x, float y, float neg_zero) { return __builtin_fmaf((float)x, y, neg_zero); }
+
+// t[e] = k[e] * q[e] for 8 f16 values in a register quad and 8 uniform f32 values. One block, so that a
+// product is never used by the very next instruction (left to itself the compiler puts a wait state there).
+__device__ __forceinline__ void mul8_f16(float (&t)[8], u32x4 k, const float* q, float neg_zero) {
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+        asm("v_fma_mix_f32 %0, %4, %6, %10 op_sel_hi:[1,0,0]\n\t"
+            "v_fma_mix_f32 %1, %4, %7, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+            "v_fma_mix_f32 %2, %5, %8, %10 op_sel_hi:[1,0,0]\n\t"
+            "v_fma_mix_f32 %3, %5, %9, %10 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+            : "=&v"(t[4 * h]), "=&v"(t[4 * h + 1]), "=&v"(t[4 * h + 2]), "=&v"(t[4 * h + 3])
+            : "v"(k[2 * h]), "v"(k[2 * h + 1]), "s"(q[4 * h]), "s"(q[4 * h + 1]), "s"(q[4 * h + 2]), "s"(q[4 * h + 3]),
+              "v"(neg_zero));
+}
+
+// attnScore with the K rows staged through LDS: one workgroup takes
+// kScoreRows rows and 4 query heads of one kv head, one wave per head and one
+// row per lane, so a row is read from memory once per 4 heads, coalesced. Each
+// dot keeps the shader's order (d = 0, 1, ...: products and sums rounded, one
+// chain per thread), and that chain is the bound: 2 VALU instructions per
+// element (the q value is uniform, read through the scalar cache). Rows are
+// padded by 16 bytes in LDS, so the lanes' 16-byte reads meet no bank conflict.
+// Measured at 8 heads, head_dim 512, 2048 rows: 113.1 us as one strided global
+// read per element and thread, 7.5 us here.
+constexpr unsigned kScoreRows = 64;
+constexpr unsigned kScoreHeads = 4;
+
+template <int HD>
+__global__ __launch_bounds__(kWG) void k_attn_score_tile(const float* __restrict__ q, const uint16_t* __restrict__ k_cache,
+                                                         float* __restrict__ scores, g4_attn_score_params p) {
+    constexpr unsigned kPieces = HD / 8;                                  // 16-byte pieces of a row
+    constexpr unsigned kStride = HD + 8;                                  // f16 elements between LDS rows
+    constexpr unsigned kLoads = kScoreRows * kPieces / kWG;               // pieces per thread
+    __shared__ f16 tile[kScoreRows * kStride];
+    const unsigned group = p.num_q_heads / p.num_kv_heads;
+    const unsigned hblocks = (group + kScoreHeads - 1) / kScoreHeads;
+    const unsigned kvh = blockIdx.y / hblocks;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const unsigned hg = (blockIdx.y % hblocks) * kScoreHeads + wave;      // head within the group
+    const unsigned row0 = blockIdx.x * kScoreRows;
+    const unsigned first = p.sliding_window != 0u && p.seq_len > p.sliding_window ? p.seq_len - p.sliding_window : 0u;
+    const unsigned pos = row0 + lane;
+    const bool live = hg < group && pos < p.seq_len;
+    float* dst = scores + (uint64_t)(kvh * group + hg) * p.seq_len + pos;
+    if (row0 + kScoreRows <= first) {  // uniform: every row of the tile is before the window
+        if (live) *dst = -1e30f;
+        return;
+    }
+    const uint64_t stride = (uint64_t)p.num_kv_heads * HD;
+    const uint16_t* krows = k_cache + (uint64_t)kvh * HD;
+    f16x8 v[kLoads];
+#pragma unroll
+    for (unsigned i = 0; i < kLoads; i++) {
+        const unsigned c = threadIdx.x + i * kWG;
+        v[i] = ldg<f16x8>(krows + min(row0 + c / kPieces, p.seq_len - 1u) * stride + (c % kPieces) * 8);
+    }
+#pragma unroll
+    for (unsigned i = 0; i < kLoads; i++) {
+        const unsigned c = threadIdx.x + i * kWG;
+        *reinterpret_cast<f16x8*>(tile + (c / kPieces) * kStride + (c % kPieces) * 8) = v[i];
+    }
+    __syncthreads();
+    if (hg >= group) return;
+    const float* __restrict__ qh = q + (uint64_t)(kvh * group + hg) * HD;
+    const f16* row = tile + lane * kStride;
+    const float nz = opaque_neg_zero();
+    // Two sets of operands in turn: a set is requested when the other has arrived (scalar loads return in
+    // any order, so only a full wait tells), and is in flight under the other's chain.
+    u32x4 ka[4], kb[4];
+    float qa[32], qb[32], dot = 0.0f;
+    auto load = [&](u32x4(&k8)[4], float(&qd)[32], unsigned d) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+#pragma unroll
+        for (unsigned i = 0; i < 4; i++) k8[i] = *reinterpret_cast<const u32x4*>(row + d + 8 * i);
+#pragma unroll
+        for (unsigned i = 0; i < 32; i++) qd[i] = qh[d + i];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto chain = [&](const u32x4(&k8)[4], const float(&qd)[32]) {
+#pragma unroll
+        for (unsigned i = 0; i < 32; i += 8) {
+            float t[8];
+            mul8_f16(t, k8[i / 8], qd + i, nz);
+#pragma unroll
+            for (unsigned e = 0; e < 8; e++) dot = dot + t[e];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load(ka, qa, 0);
+    for (unsigned d = 0; d < HD; d += 64) {
+        load(kb, qb, d + 32);
+        chain(ka, qa);
+        load(ka, qa, (d + 64) % HD);
+        chain(kb, qb);
+    }
+    if (live) *dst = pos < first ? -1e30f : dot * p.scale;
+}
+
 __global__ __launch_bounds__(kWG) void k_softmax(float* __restrict__ scores, g4_softmax_params p) {
     __shared__ float shared_max[kWG];
     __shared__ float shared_sum[kWG];
@@ -100,6 +213,63 @@ __global__ __launch_bounds__(kWG) void k_softmax(float* __restrict__ scores, g4_
     for (unsigned i = tid; i < p.seq_len; i += kWG) scores[base + i] = scores[base + i] / sum_val;
 }
 
+// softmax of heads of up to 1024 R scores: each thread keeps its R scores in
+// registers, so memory is read and written once (the loop form above passes over
+// it three times, a memory round trip per pass and 256 scores), and 1024 threads
+// share the f64 exponentials. The sum keeps the shader's order: exponentials pass
+// through LDS to the 256 partials, each added in index order, then the 128 -> 1
+// tree. Bound by its chain of latencies. Measured at 8 heads of 2048 scores:
+// 8.2 us -> 5.0 us.
+constexpr unsigned kSoftThreads = 1024;
+
+template <int R>
+__global__ __launch_bounds__(kSoftThreads) void k_softmax_reg(float* __restrict__ scores, g4_softmax_params p) {
+    __shared__ float e_all[kSoftThreads * R];
+    __shared__ float red[kWG + 1];
+    const unsigned tid = threadIdx.x;
+    float* base = scores + (uint64_t)blockIdx.x * p.seq_len;
+    float x[R];
+    float local_max = -1e30f;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const unsigned i = tid + r * kSoftThreads;
+        x[r] = i < p.seq_len ? base[i] : -1e30f;
+        local_max = wgsl_max(local_max, x[r]);
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) local_max = wgsl_max(local_max, __shfl_xor(local_max, m));  // no NaN: any order
+    if ((tid & 63) == 0) red[tid >> 6] = local_max;
+    __syncthreads();
+    float max_val = red[0];
+#pragma unroll
+    for (unsigned w = 1; w < kSoftThreads / 64; w++) max_val = wgsl_max(max_val, red[w]);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const unsigned i = tid + r * kSoftThreads;
+        x[r] = (float)exp((double)(x[r] - max_val));
+        if (i < p.seq_len) e_all[i] = x[r];
+    }
+    __syncthreads();  // also: every thread has read the wave maxima
+    if (tid < kWG) {
+        float sum = 0.0f;
+        for (unsigned i = tid; i < p.seq_len; i += kWG) sum = sum + e_all[i];
+        red[tid] = sum;
+    }
+    __syncthreads();
+    if (tid < 64) {  // strides 128, 64, then 32 .. 1 within the wave: wg_tree_sum's operand pairs
+        float s = (red[tid] + red[tid + 128]) + (red[tid + 64] + red[tid + 192]);
+        s = wave_tree_sum(s);
+        if (tid == 0) red[kWG] = s;
+    }
+    __syncthreads();
+    const float sum_val = red[kWG];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const unsigned i = tid + r * kSoftThreads;
+        if (i < p.seq_len) base[i] = x[r] / sum_val;
+    }
+}
+
 __global__ __launch_bounds__(kWG) void k_attn_output(const float* __restrict__ probs,
                                                      const uint16_t* __restrict__ v_cache, float* __restrict__ out,
                                                      g4_attn_output_params p) {
@@ -117,6 +287,142 @@ __global__ __launch_bounds__(kWG) void k_attn_output(const float* __restrict__ p
         sum = sum + prob * h2f(v_cache[v_idx]);
     }
     out[(uint64_t)head * p.head_dim + d] = sum;
+}
+
+// attnOutput for head_dims of whole 64-column blocks. An output's sum is one
+// chain over the rows (each product and sum rounded, in row order), so what
+// bounds the kernel is the chain's length; the form above puts two dependent
+// loads, a conversion and a product on every link. Here the workgroup's wave 0
+// holds the 64 chains and does nothing but add: the other seven waves read
+// V and the probabilities two rounds ahead (16 bytes a lane, 8 rows a load),
+// multiply, and leave the products in LDS, four rows of a column side by side
+// (one 16-byte read per four additions).
+// A block of rows whose products are all zero is not added: the sum starts at +0
+// and never becomes -0, so adding a zero of either sign returns its bits (rows
+// before a sliding window have probability 0; 0 * inf is NaN and is added).
+// Measured at 8 heads, head_dim 512, 2048 rows: 502.3 us -> 12.8 us.
+constexpr unsigned kOutMul = 7;    // multiplying waves
+constexpr unsigned kOutRows = 32;  // rows of a multiplying wave per round
+constexpr unsigned kOutRound = kOutMul * kOutRows;
+constexpr unsigned kOutQuad = 288;  // floats of 4 rows of products: 8 groups of 8 columns x 4 rows, 4 floats between
+                                    // groups (the multiplying lanes' 64 stores then fall in 64 different banks)
+
+struct OutSmem {
+    f32x4 prod[2][kOutMul][kOutRows / 4][kOutQuad / 4];  // [round parity][wave][row / 4]
+    uint32_t live[2][kOutMul];                           // some product of the block is not zero
+};
+
+// A multiplying wave's operands of one round: lane (r, c) = 8 r + c holds rows 8 i + r, columns 8 c .. + 7.
+struct OutRows {
+    f16x8 v[kOutRows / 8];
+    float p[kOutRows / 8];
+};
+
+__device__ __forceinline__ void out_load(OutRows& x, const uint16_t* v, uint64_t stride, const float* probs, unsigned row0,
+                                         unsigned rows, unsigned lane) {
+#pragma unroll
+    for (unsigned i = 0; i < kOutRows / 8; i++) {
+        const unsigned row = min(row0 + 8 * i + (lane >> 3), rows - 1);  // clamped: see out_multiply
+        x.p[i] = ldg<float>(probs + row);
+        x.v[i] = ldg<f16x8>(v + row * stride + (lane & 7) * 8);
+    }
+}
+
+__device__ __forceinline__ void out_multiply(const OutRows& x, OutSmem& sm, unsigned par, unsigned wave, unsigned lane,
+                                             unsigned row0, unsigned rows, float nz) {
+    uint32_t any = 0;
+#pragma unroll
+    for (unsigned i = 0; i < kOutRows / 8; i++) {
+        const unsigned r = 8 * i + (lane >> 3);
+        const bool in = row0 + r < rows;  // rows past the end: 0 * 0, which adds +0
+        const float p = in ? x.p[i] : 0.0f;
+        const f16x8 v = in ? x.v[i] : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        float* dst = reinterpret_cast<float*>(sm.prod[par][wave][r / 4]) + (lane & 7) * 36 + r % 4;
+#pragma unroll
+        for (unsigned e = 0; e < 8; e++) {
+            const float y = mul_f16(v[e], p, nz);
+            any |= __float_as_uint(y);
+            dst[4 * e] = y;
+        }
+    }
+    const bool nonzero = __any((any << 1) != 0);
+    if (lane == 0) sm.live[par][wave] = nonzero;
+}
+
+__global__ __launch_bounds__(64 * (kOutMul + 1)) void k_attn_output_chain(const float* __restrict__ probs,
+                                                                          const uint16_t* __restrict__ v_cache,
+                                                                          float* __restrict__ out,
+                                                                          g4_attn_output_params p) {
+    __shared__ OutSmem sm;
+    const unsigned lane = threadIdx.x & 63;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned head = blockIdx.y, d = blockIdx.x * 64 + lane, rows = p.seq_len;
+    const unsigned kv_head = head / (p.num_q_heads / p.num_kv_heads);
+    const uint64_t stride = (uint64_t)p.num_kv_heads * p.head_dim;
+    const unsigned rounds = (rows + kOutRound - 1) / kOutRound;
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(3);  // one multiplying wave shares its SIMD
+        float sum = 0.0f;
+        for (unsigned t = 0; t < rounds; t++) {
+            __syncthreads();
+            const unsigned par = t & 1;
+            uint64_t todo = __ballot(lane < kOutMul && sm.live[par][min(lane, kOutMul - 1)] != 0);
+            if (!todo) continue;  // uniform, as every branch here
+            f32x4 x[kOutRows / 4], y[kOutRows / 4];  // a block is read from LDS under the additions of the one before
+            auto take = [&](f32x4(&to)[kOutRows / 4]) {
+                const unsigned w = (unsigned)__builtin_ctzll(todo);
+#pragma unroll
+                for (unsigned r = 0; r < kOutRows / 4; r++) to[r] = sm.prod[par][w][r][lane + lane / 8];
+                todo &= todo - 1;
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto add = [&](const f32x4(&from)[kOutRows / 4]) {
+#pragma unroll
+                for (unsigned r = 0; r < kOutRows / 4; r++)
+#pragma unroll
+                    for (unsigned e = 0; e < 4; e++) sum = sum + from[r][e];
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            take(x);
+            while (true) {
+                if (!todo) {
+                    add(x);
+                    break;
+                }
+                take(y);
+                add(x);
+                if (!todo) {
+                    add(y);
+                    break;
+                }
+                take(x);
+                add(y);
+            }
+        }
+        out[(uint64_t)head * p.head_dim + d] = sum;
+        return;
+    }
+    const unsigned mw = wave - 1;
+    const uint16_t* v = v_cache + (uint64_t)kv_head * p.head_dim + blockIdx.x * 64;
+    const float* pr = probs + (uint64_t)head * rows;
+    const float nz = opaque_neg_zero();
+    OutRows a, b;
+    unsigned row0 = mw * kOutRows;
+    out_load(a, v, stride, pr, row0, rows, lane);
+    out_load(b, v, stride, pr, row0 + kOutRound, rows, lane);
+    // Barrier t (the adding wave's t-th) follows the multiplication of round t; a buffer is written
+    // again after the next barrier, which the adding wave reaches when it is done with it.
+    for (unsigned t = 0; t < rounds; t += 2) {
+        out_multiply(a, sm, 0, mw, lane, row0, rows, nz);
+        out_load(a, v, stride, pr, row0 + 2 * kOutRound, rows, lane);
+        __syncthreads();
+        if (t + 1 < rounds) {  // uniform
+            out_multiply(b, sm, 1, mw, lane, row0 + kOutRound, rows, nz);
+            out_load(b, v, stride, pr, row0 + 3 * kOutRound, rows, lane);
+            __syncthreads();
+        }
+        row0 += 2 * kOutRound;
+    }
 }
 
 __global__ __launch_bounds__(kWG) void k_zero(uint32_t* __restrict__ dst, uint64_t words, uint8_t* tail,
@@ -176,6 +482,18 @@ int g4_attn_score(const float* q, const uint16_t* k_cache, float* scores, g4_att
                     p.num_kv_heads);
     const uint64_t total = (uint64_t)p.num_q_heads * p.seq_len;
     if (total == 0) return G4_OK;
+    const unsigned group = p.num_q_heads / p.num_kv_heads;
+    const uint64_t hblocks = (uint64_t)p.num_kv_heads * ((group + kScoreHeads - 1) / kScoreHeads);
+    // The tile form: the head_dims it is built for, 16-byte K rows, and a grid within the launch limit.
+    if ((p.head_dim == 256 || p.head_dim == 512) && !(reinterpret_cast<uintptr_t>(k_cache) & 15) && hblocks <= 65535) {
+        const dim3 grid(ceil_div_u(p.seq_len, kScoreRows), (unsigned)hblocks);
+        if (p.head_dim == 256)
+            G4_LAUNCH(k_attn_score_tile<256>, grid, dim3(kWG), 0, as_stream(stream), q, k_cache, scores, p);
+        else
+            G4_LAUNCH(k_attn_score_tile<512>, grid, dim3(kWG), 0, as_stream(stream), q, k_cache, scores, p);
+        G4_CHECK_LAUNCH("attnScore");
+        return G4_OK;
+    }
     G4_LAUNCH(k_attn_score, dim3(ceil_div_u(total, kWG)), dim3(kWG), 0, as_stream(stream), q, k_cache,
                        scores, p);
     G4_CHECK_LAUNCH("attnScore");
@@ -186,6 +504,16 @@ int g4_softmax(float* scores, g4_softmax_params p, void* stream) {
     if (!scores) return fail(G4_EINVAL, "softmax: NULL scores");
     if (p.seq_len == 0) return fail(G4_EINVAL, "softmax: seq_len 0");
     if (p.num_heads == 0) return G4_OK;
+    if (p.seq_len <= 4 * kSoftThreads) {
+        G4_LAUNCH(k_softmax_reg<4>, dim3(p.num_heads), dim3(kSoftThreads), 0, as_stream(stream), scores, p);
+        G4_CHECK_LAUNCH("softmax");
+        return G4_OK;
+    }
+    if (p.seq_len <= 16 * kSoftThreads) {  // up to the scores that LDS and the registers hold
+        G4_LAUNCH(k_softmax_reg<16>, dim3(p.num_heads), dim3(kSoftThreads), 0, as_stream(stream), scores, p);
+        G4_CHECK_LAUNCH("softmax");
+        return G4_OK;
+    }
     G4_LAUNCH(k_softmax, dim3(p.num_heads), dim3(kWG), 0, as_stream(stream), scores, p);
     G4_CHECK_LAUNCH("softmax");
     return G4_OK;
@@ -198,6 +526,13 @@ int g4_attn_output(const float* probs, const uint16_t* v_cache, float* out, g4_a
                     p.num_kv_heads);
     const uint64_t total = (uint64_t)p.num_q_heads * p.head_dim;
     if (total == 0) return G4_OK;
+    if (p.head_dim % 64 == 0 && p.seq_len > 0 && p.seq_len < 0x40000000u && p.num_q_heads <= 65535 &&
+        !(reinterpret_cast<uintptr_t>(v_cache) & 15)) {
+        G4_LAUNCH(k_attn_output_chain, dim3(p.head_dim / 64, p.num_q_heads), dim3(64 * (kOutMul + 1)), 0,
+                  as_stream(stream), probs, v_cache, out, p);
+        G4_CHECK_LAUNCH("attnOutput");
+        return G4_OK;
+    }
     G4_LAUNCH(k_attn_output, dim3(ceil_div_u(total, kWG)), dim3(kWG), 0, as_stream(stream), probs, v_cache,
                        out, p);
     G4_CHECK_LAUNCH("attnOutput");
