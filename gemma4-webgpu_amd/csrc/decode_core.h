@@ -181,15 +181,22 @@ __device__ __forceinline__ void store_q_chunk(DecodeSmem<HD, W>& sm, int c, int 
 // Tile loads. K in score-operand layout: lane (n, g) holds K[row n][32c + 8g .. +8].
 // Offsets are 32-bit bytes from the wave-uniform cache base of the kv head
 // (caches are limited to 4 GiB on the host), so loads use an SGPR base and a
-// VGPR offset. Rows beyond `last` are clamped to it.
-template <int HD>
+// VGPR offset. Rows beyond `last` are clamped to it. kStream: non-temporal
+// (rows read once); otherwise the L2 keeps the rows for other workgroups.
+template <bool kStream, typename T>
+__device__ __forceinline__ T ldg_row(const void* p) {
+    if constexpr (kStream) return ldg_stream<T>(p);
+    return ldg<T>(p);
+}
+
+template <int HD, bool kStream = true>
 __device__ __forceinline__ void load_k_tile(const char* Kb, uint32_t row_bytes, unsigned last, int n, int g, unsigned kt0,
                                             f16x8 (&kr)[2][DecodeDims<HD>::NC]) {
 #pragma unroll
     for (int h2 = 0; h2 < 2; h2++) {
         const uint32_t off = min(kt0 + h2 * 16 + n, last) * row_bytes + (uint32_t)g * 16u;
 #pragma unroll
-        for (int c = 0; c < DecodeDims<HD>::NC; c++) kr[h2][c] = ldg_stream<f16x8>(Kb + (off + c * 64u));
+        for (int c = 0; c < DecodeDims<HD>::NC; c++) kr[h2][c] = ldg_row<kStream, f16x8>(Kb + (off + c * 64u));
     }
 }
 
@@ -197,14 +204,14 @@ __device__ __forceinline__ void load_k_tile(const char* Kb, uint32_t row_bytes, 
 // row(g, t) = 4g + t for t < 4, 16 + 4g + (t - 4) otherwise.
 __device__ __forceinline__ unsigned v_row(int g, int t) { return t < 4 ? g * 4 + t : 16 + g * 4 + (t - 4); }
 
-template <int HD>
+template <int HD, bool kStream = true>
 __device__ __forceinline__ void load_v_tile(const char* Vb, uint32_t row_bytes, unsigned last, int n, int g, unsigned kt0,
                                             u32x4 (&vr)[DecodeDims<HD>::NB][8]) {
 #pragma unroll
     for (int t = 0; t < 8; t++) {
         const uint32_t off = min(kt0 + v_row(g, t), last) * row_bytes + (uint32_t)n * 16u;
 #pragma unroll
-        for (int b = 0; b < DecodeDims<HD>::NB; b++) vr[b][t] = ldg_stream<u32x4>(Vb + (off + b * 256u));
+        for (int b = 0; b < DecodeDims<HD>::NB; b++) vr[b][t] = ldg_row<kStream, u32x4>(Vb + (off + b * 256u));
     }
 }
 

@@ -89,7 +89,10 @@ struct StepSmem {
 // parts move with its first attended row (step_part_rows), and the RoPE
 // factors are evaluated here from the inverse frequencies of the entry's set,
 // in f64 rounded to f32 as the host evaluates the prepared position's.
-template <int W, int HD>
+//
+// KEEP: K and V rows are read with ordinary loads, which the caches keep, and
+// not as a stream (StepPlanHost::keep_rows has the rule).
+template <int W, int HD, bool KEEP>
 __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ work, float* part_ml, float* part_o,
                                                uint32_t num_kv_heads, uint32_t group, uint32_t adv, unsigned wg,
                                                unsigned kvh, StepSmem<W, HD>& sm) {
@@ -184,9 +187,12 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
         const char* Vb = reinterpret_cast<const char*>(ent.v_cache + (uint64_t)kvh * HD);
         f16x8 kreg[2][D::NC];
         u32x4 vreg[D::NB][8];
+        auto load_tile = [&] {  // the tile at t0
+            load_k_tile<HD, !KEEP>(Kb, row_bytes, last, n, g, k0 + t0, kreg);
+            load_v_tile<HD, !KEEP>(Vb, row_bytes, last, n, g, k0 + t0, vreg);
+        };
         if constexpr (kTile) {
-            load_k_tile<HD>(Kb, row_bytes, last, n, g, k0 + t0, kreg);
-            load_v_tile<HD>(Vb, row_bytes, last, n, g, k0 + t0, vreg);
+            load_tile();
         }
         __builtin_amdgcn_sched_barrier(0);  // keep every request above ahead of the arithmetic below
 
@@ -262,8 +268,7 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
         if constexpr (kTile) {  // the first tile was requested above; the loop requests its own
             tile_step<HD>(sm.dec, lane, g, lo_col, k0 + t0, k1t, kreg, vreg, m_run, l_run, acc);
             for (t0 += kStride; t0 < nkeys; t0 += kStride) {
-                load_k_tile<HD>(Kb, row_bytes, last, n, g, k0 + t0, kreg);
-                load_v_tile<HD>(Vb, row_bytes, last, n, g, k0 + t0, vreg);
+                load_tile();
                 tile_step<HD>(sm.dec, lane, g, lo_col, k0 + t0, k1t, kreg, vreg, m_run, l_run, acc);
             }
         }
@@ -285,12 +290,12 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
     wg_combine_write<HD>(sm.dec, G, false, nullptr, a.part_o + rec * HD, a.part_ml + rec * 2, em, ev);
 }
 
-template <int W, int HD>
+template <int W, int HD, bool KEEP>
 __global__ __launch_bounds__(64 * W, HD == 256 ? 8 / W : 1) void k_attn_step(
     const StepWorkDev* __restrict__ work, float* part_ml, float* part_o, uint32_t num_kv_heads, uint32_t group,
     uint32_t adv) {
     __shared__ StepSmem<W, HD> sm;
-    attn_step_body<W, HD>(work, part_ml, part_o, num_kv_heads, group, adv, blockIdx.x, blockIdx.y, sm);
+    attn_step_body<W, HD, KEEP>(work, part_ml, part_o, num_kv_heads, group, adv, blockIdx.x, blockIdx.y, sm);
 }
 
 // Two plans of one token in one launch (E2B's two head_dim groups): the
@@ -302,6 +307,7 @@ union StepPairSmem {
     StepSmem<4, 256> b;
 };
 
+template <bool KEEP>
 __global__ __launch_bounds__(256, 1) void k_attn_step_pair(
     const StepWorkDev* __restrict__ work_a, float* ml_a, float* o_a, uint32_t nkh_a, uint32_t group_a, uint32_t adv_a,
     uint32_t wgs_a, const StepWorkDev* __restrict__ work_b, float* ml_b, float* o_b, uint32_t nkh_b, uint32_t group_b,
@@ -309,9 +315,9 @@ __global__ __launch_bounds__(256, 1) void k_attn_step_pair(
     __shared__ StepPairSmem sm;
     const unsigned x = blockIdx.x, y = blockIdx.y;
     if (x < wgs_a) {  // uniform
-        if (y < nkh_a) attn_step_body<4, 512>(work_a, ml_a, o_a, nkh_a, group_a, adv_a, x, y, sm.a);
+        if (y < nkh_a) attn_step_body<4, 512, KEEP>(work_a, ml_a, o_a, nkh_a, group_a, adv_a, x, y, sm.a);
     } else if (y < nkh_b) {
-        attn_step_body<4, 256>(work_b, ml_b, o_b, nkh_b, group_b, adv_b, x - wgs_a, y, sm.b);
+        attn_step_body<4, 256, KEEP>(work_b, ml_b, o_b, nkh_b, group_b, adv_b, x - wgs_a, y, sm.b);
     }
 }
 
@@ -341,6 +347,7 @@ struct StepPlanRep {
     uint32_t adv;        // tokens advanced since the prepare (g4_attn_step_advance)
     uint32_t max_rows;   // the largest seq_len of the prepared entries
     uint32_t max_pos;    // the largest position of the prepared entries
+    uint32_t keep_rows;  // K and V rows read with ordinary loads (StepPlanHost::keep_rows)
 };
 static_assert(sizeof(StepPlanRep) <= sizeof(g4_decode_plan), "plan size");
 static_assert(kStepMaxWgs <= 65535 && kMaxGroup <= 255, "plan field widths");
@@ -381,6 +388,7 @@ static void write_plan(g4_decode_plan* plan, char* tables, char* part_ml, const 
     r.waves = (uint8_t)ph.waves;
     r.head_dim = head_dim;
     r.magic = kStepMagic;
+    r.keep_rows = ph.keep_rows;
     r.off_merge = (uint32_t)ph.off_merge;
     r.off_rope = (uint32_t)ph.off_rope;
     r.off_ents = (uint32_t)ph.off_ents;
@@ -496,28 +504,19 @@ static int launch_attention(const g4_decode_plan* plan, void* stream, hipEvent_t
     const dim3 grid(r.n_wgs, r.num_kv_heads);
     hipStream_t st = as_stream(stream);
     const uint32_t adv = r.adv;
-    if (r.head_dim == 512) {
+    auto launch = [&](auto kernel, unsigned threads) {
         if (start || stop)
-            hipExtLaunchKernelGGL((k_attn_step<4, 512>), grid, dim3(256), 0, st, start, stop, 0, a.work, a.part_ml,
-                                  a.part_o, a.num_kv_heads, a.group, adv);
+            hipExtLaunchKernelGGL(kernel, grid, dim3(threads), 0, st, start, stop, 0, a.work, a.part_ml, a.part_o,
+                                  a.num_kv_heads, a.group, adv);
         else
-            G4_LAUNCH((k_attn_step<4, 512>), grid, dim3(256), 0, st, a.work, a.part_ml, a.part_o, a.num_kv_heads,
-                      a.group, adv);
-    } else if (r.waves == 8) {
-        if (start || stop)
-            hipExtLaunchKernelGGL((k_attn_step<8, 256>), grid, dim3(512), 0, st, start, stop, 0, a.work, a.part_ml,
-                                  a.part_o, a.num_kv_heads, a.group, adv);
-        else
-            G4_LAUNCH((k_attn_step<8, 256>), grid, dim3(512), 0, st, a.work, a.part_ml, a.part_o, a.num_kv_heads,
-                      a.group, adv);
-    } else {
-        if (start || stop)
-            hipExtLaunchKernelGGL((k_attn_step<4, 256>), grid, dim3(256), 0, st, start, stop, 0, a.work, a.part_ml,
-                                  a.part_o, a.num_kv_heads, a.group, adv);
-        else
-            G4_LAUNCH((k_attn_step<4, 256>), grid, dim3(256), 0, st, a.work, a.part_ml, a.part_o, a.num_kv_heads,
-                      a.group, adv);
-    }
+            G4_LAUNCH(kernel, grid, dim3(threads), 0, st, a.work, a.part_ml, a.part_o, a.num_kv_heads, a.group, adv);
+    };
+    if (r.head_dim == 512)
+        r.keep_rows ? launch(k_attn_step<4, 512, true>, 256) : launch(k_attn_step<4, 512, false>, 256);
+    else if (r.waves == 8)
+        r.keep_rows ? launch(k_attn_step<8, 256, true>, 512) : launch(k_attn_step<8, 256, false>, 512);
+    else
+        r.keep_rows ? launch(k_attn_step<4, 256, true>, 256) : launch(k_attn_step<4, 256, false>, 256);
     G4_CHECK_LAUNCH("attnStep");
     return G4_OK;
 }
@@ -544,14 +543,16 @@ static int launch_attention_pair(const g4_decode_plan* plan_1, const g4_decode_p
     const StepWorkDev* wa = reinterpret_cast<const StepWorkDev*>(a.tables);
     const StepWorkDev* wb = reinterpret_cast<const StepWorkDev*>(b.tables);
     hipStream_t st = as_stream(stream);
-    if (start || stop)
-        hipExtLaunchKernelGGL(k_attn_step_pair, grid, dim3(256), 0, st, start, stop, 0, wa, ml(a), po(a),
-                              (uint32_t)a.num_kv_heads, (uint32_t)a.group, a.adv, (uint32_t)a.n_wgs, wb, ml(b), po(b),
-                              (uint32_t)b.num_kv_heads, (uint32_t)b.group, b.adv);
-    else
-        G4_LAUNCH(k_attn_step_pair, grid, dim3(256), 0, st, wa, ml(a), po(a), (uint32_t)a.num_kv_heads,
-                  (uint32_t)a.group, a.adv, (uint32_t)a.n_wgs, wb, ml(b), po(b), (uint32_t)b.num_kv_heads,
-                  (uint32_t)b.group, b.adv);
+    auto launch = [&](auto kernel) {
+        if (start || stop)
+            hipExtLaunchKernelGGL(kernel, grid, dim3(256), 0, st, start, stop, 0, wa, ml(a), po(a),
+                                  (uint32_t)a.num_kv_heads, (uint32_t)a.group, a.adv, (uint32_t)a.n_wgs, wb, ml(b),
+                                  po(b), (uint32_t)b.num_kv_heads, (uint32_t)b.group, b.adv);
+        else
+            G4_LAUNCH(kernel, grid, dim3(256), 0, st, wa, ml(a), po(a), (uint32_t)a.num_kv_heads, (uint32_t)a.group,
+                      a.adv, (uint32_t)a.n_wgs, wb, ml(b), po(b), (uint32_t)b.num_kv_heads, (uint32_t)b.group, b.adv);
+    };
+    a.keep_rows || b.keep_rows ? launch(k_attn_step_pair<true>) : launch(k_attn_step_pair<false>);
     G4_CHECK_LAUNCH("attnStepPair");
     return G4_OK;
 }

@@ -28,6 +28,7 @@ namespace g4 {
 // workgroups fit one wave of the GPU (at most kStepMaxWgs), so at most that
 // many records exist.
 constexpr unsigned kStepMaxWgs = 1024;
+constexpr unsigned kXcds = 8;            // workgroups go round the XCDs in index order
 constexpr unsigned kStepOneWgTiles = 16;  // one workgroup per CU up to this many tiles each
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -100,6 +101,13 @@ struct StepPlanHost {
     uint32_t n_wgs = 0;      // workgroups (work items)
     uint32_t n_merge = 0;    // entries in the merge table
     uint32_t max_parts = 0;  // largest part count of an entry
+    // The attention kernel reads rows with ordinary loads: where entries share rows
+    // (a row is read again, from L2 or the MALL). Otherwise a row is read once per
+    // token and streamed: a step larger than the MALL is faster so (64 sequences of
+    // 1K to 32K rows 188 us streamed, 204 kept), and a smaller one does not write back
+    // what earlier work left dirty there (35 layers at 8192, caches full of written
+    // lines: 23.6 us streamed, 34.9 kept; full of read ones: 23.2 and 22.5).
+    bool keep_rows = false;
     uint32_t parts = 0;      // partial-record slots in use
     size_t off_merge = 0;    // byte offsets in the tables blob
     size_t off_ents = 0;
@@ -112,6 +120,8 @@ struct StepPlanHost {
     std::vector<std::pair<const float*, uint32_t>> rope_keys;
     std::vector<const float*> rope_dev;  // device address of each distinct pair's factors
     std::vector<uint32_t> rope_set;      // its set in this blob, or ~0 when an earlier plan placed it
+    std::vector<uint32_t> part_base;               // first partial record of an entry
+    std::vector<uint32_t> kv_slot, kv_first, kv_next;  // entries that read the same rows (see kv_groups)
 };
 
 // Hash of an (inverse-frequency table, position) pair.
@@ -243,6 +253,41 @@ inline uint32_t rope_pair_index(StepPlanHost& ph, const float* table, uint32_t p
         }
         if (ph.rope_keys[v - 1].first == table && ph.rope_keys[v - 1].second == position) return v - 1;
     }
+}
+
+// Groups the entries that read the same cache rows (KV-sharing layers of one
+// token): kv_first[i] is the first entry with entry i's caches and row range,
+// kv_next[i] the next one of its group (~0: the last). Returns whether any
+// group has two entries. Open addressing as in rope_pair_index.
+inline bool kv_groups(StepPlanHost& ph) {
+    const uint32_t n = (uint32_t)ph.tab.size();
+    size_t slots = 16;
+    while (slots < 2 * (size_t)n) slots *= 2;
+    ph.kv_slot.assign(slots, 0u);
+    ph.kv_first.resize(n);
+    ph.kv_next.assign(n, ~0u);
+    bool shared = false;
+    for (uint32_t i = 0; i < n; i++) {
+        const StepEntryDev& e = ph.tab[i];
+        const uint64_t h = (reinterpret_cast<uintptr_t>(e.k_cache) >> 4) * 0x9E3779B97F4A7C15ull ^
+                           e.key_end * 0xC2B2AE3D27D4EB4Full;
+        for (size_t s = (size_t)(h >> 32) & (slots - 1);; s = (s + 1) & (slots - 1)) {
+            const uint32_t v = ph.kv_slot[s];  // 0 = empty, else the group's latest entry + 1
+            if (v) {
+                const StepEntryDev& f = ph.tab[v - 1];
+                if (f.k_cache != e.k_cache || f.v_cache != e.v_cache || f.key_end != e.key_end || f.window != e.window)
+                    continue;
+                ph.kv_first[i] = ph.kv_first[v - 1];
+                ph.kv_next[v - 1] = i;
+                shared = true;
+            } else {
+                ph.kv_first[i] = i;
+            }
+            ph.kv_slot[s] = i + 1;
+            break;
+        }
+    }
+    return shared;
 }
 
 // Checks the step's arguments and plans it. `tables` is the device address of
@@ -401,19 +446,48 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
             if (share) share->add(ph.rope_keys[k], ph.rope_dev[k]);
         }
     }
-    // Work items entry by entry (each with a copy of its entry), the merge
-    // table and the entry table (every entry: attnOut, first record, parts).
+    // The merge table and the entry table (every entry: attnOut, first record, parts).
     StepWorkDev* work = reinterpret_cast<StepWorkDev*>(blob);
     DecodeEntryDev* merge = reinterpret_cast<DecodeEntryDev*>(blob + off_merge);
     DecodeEntryDev* ents = reinterpret_cast<DecodeEntryDev*>(blob + off_ents);
     uint32_t part_next = 0;
+    const bool shared = kv_groups(ph);
+    ph.part_base.resize(n_entries);
     for (uint32_t i = 0; i < n_entries; i++) {
         StepEntryDev& d = ph.tab[i];
         if (ph.rope_idx[i] != ~0u) d.rope_cs = ph.rope_dev[ph.rope_idx[i]];
-        const uint64_t ne = tiles[i], we = d.n_parts;
+        const uint64_t we = d.n_parts;
         const uint32_t part_base = we > 1 ? part_next : 0;
+        ph.part_base[i] = part_base;
+        if (we > 1) {
+            part_next += (uint32_t)we;
+            *merge++ = DecodeEntryDev{nullptr, nullptr, nullptr, d.out, 0, 0, part_base, (uint32_t)we, 0.0f, 0};
+        }
+        ents[i] = DecodeEntryDev{nullptr, nullptr, nullptr, d.out, 0, 0, part_base, (uint32_t)we, 0.0f, 0};
+    }
+    // Work items, in the order of the workgroups that take them: entry by entry,
+    // part by part. Workgroup w runs on XCD w % 8, each with its own L2, so when
+    // entries share cache rows the items of one part of a group (the same rows,
+    // different queries) take consecutive workgroups of one XCD: its L2 then reads
+    // those rows once for most of them. Measured on a token of E2B's real shapes
+    // (us, one state / three in turn): position 32768 81.0 / 85.9 entry by entry
+    // with streaming loads, 78.2 in this order, 70.4 / 76.6 in this order with
+    // ordinary loads; 16384 56.0 -> 41.6; 8192 37.3 -> 30.6; 2048 23.0 -> 21.1.
+    size_t at = 0, xcd = 0;
+    auto next_item = [&]() -> StepWorkDev& {
+        StepWorkDev& w = work[at];
+        if (!shared) {
+            at++;
+        } else if ((at += kXcds) >= n_work) {
+            at = ++xcd;
+        }
+        return w;
+    };
+    for (uint32_t i = 0; i < n_entries; i++) {
+        if (shared && ph.kv_first[i] != i) continue;  // placed with its group
         // Part j covers tiles [j ne / we, (j + 1) ne / we): the bounds advance by
         // ne / we and carry the remainder, with no division per part.
+        const uint64_t ne = tiles[i], we = ph.tab[i].n_parts;
         const uint64_t step = ne / we, rem = ne % we;
         uint64_t te = 0, acc = 0;
         for (uint64_t j = 0; j < we; j++) {
@@ -426,19 +500,17 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
             }
             const uint64_t rb = key_begin[i] + tb * kTileKeys;
             const uint64_t re = key_begin[i] + te * kTileKeys;
-            StepWorkDev& w = *work++;
-            w.ent = d;
-            w.row_begin = (uint32_t)rb;
-            w.row_end = (uint32_t)(re < d.key_end ? re : d.key_end);
-            w.part = we > 1 ? part_base + (uint32_t)j : 0u;
-            w.entry = i;
+            for (uint32_t m = i; m != ~0u; m = shared ? ph.kv_next[m] : ~0u) {  // the same rows, hence the same parts
+                StepWorkDev& w = next_item();
+                w.ent = ph.tab[m];
+                w.row_begin = (uint32_t)rb;
+                w.row_end = (uint32_t)(re < w.ent.key_end ? re : w.ent.key_end);
+                w.part = we > 1 ? ph.part_base[m] + (uint32_t)j : 0u;
+                w.entry = m;
+            }
         }
-        if (we > 1) {
-            part_next += (uint32_t)we;
-            *merge++ = DecodeEntryDev{nullptr, nullptr, nullptr, d.out, 0, 0, part_base, (uint32_t)we, 0.0f, 0};
-        }
-        ents[i] = DecodeEntryDev{nullptr, nullptr, nullptr, d.out, 0, 0, part_base, (uint32_t)we, 0.0f, 0};
     }
+    ph.keep_rows = shared;
     ph.waves = waves;
     ph.n_wgs = (uint32_t)n_work;
     ph.n_merge = n_merge;
