@@ -20,11 +20,18 @@ from .abi import (G4_WEIGHT_Q4K, G4_WEIGHT_Q8, AttnOutputParams, AttnScoreParams
                   MatmulParams, NormParams, NormRopeParams, PrepLayer, PrepParams, SoftcapParams, SoftmaxParams,
                   StepEntry, PromptPrepParams)
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
 F16_TYPES = (torch.float16, torch.int16, torch.uint16)
 
 
 def _stream(stream=None) -> int:
     if stream is None:
+        # The current stream's handle itself where torch gives it (0.2 us): current_stream builds a Stream
+        # object first (3.1 us of the 7.7 us that a call took, kernel launch included).
+        if _raw_stream is not None and torch.cuda.is_initialized():
+            return _raw_stream(_current_device())
         stream = torch.cuda.current_stream()
     return int(stream.cuda_stream) if hasattr(stream, "cuda_stream") else int(stream)
 
@@ -32,10 +39,11 @@ def _stream(stream=None) -> int:
 def _dev(t: torch.Tensor, name: str, dtypes, min_numel: int) -> int:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name}: expected a tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name}: must be on the GPU, got {t.device}")
-    if t.dtype not in (dtypes if isinstance(dtypes, tuple) else (dtypes,)):
-        raise TypeError(f"{name}: dtype {t.dtype} not in {dtypes}")
+    dtype = t.dtype
+    if dtype is not dtypes and dtype not in (dtypes if isinstance(dtypes, tuple) else (dtypes,)):
+        raise TypeError(f"{name}: dtype {dtype} not in {dtypes}")
     if not t.is_contiguous():
         raise ValueError(f"{name}: must be contiguous")
     if t.numel() < min_numel:
