@@ -35,7 +35,6 @@ struct LinearArgs {
     LinearSegDev seg[kLinearMaxSegs];
     uint32_t n_segs;
     uint32_t total_rows;
-    uint32_t rows_per_wave;  // even
 };
 
 template <int FMT, int NJ>
@@ -51,27 +50,54 @@ __device__ __forceinline__ float linear_row(const LinearSegDev& sg, unsigned lr,
         return gemv_row_dot<NJ, false>(static_cast<const uint16_t*>(sg.w) + (uint64_t)lr * N, xr, lq);
 }
 
-template <int FMT, int NJ>
-__global__ __launch_bounds__(256) void k_linear(LinearArgs a) {
+// What a wave needs before its first request comes as scalars that are preloaded
+// into SGPRs at wave start (the file is compiled with kernarg preloading): the
+// input, the first three weight matrices with the rows they begin at, and the
+// rows per wave. The rest (outputs, scales, a fourth matrix) is read from the
+// argument memory under the first weight loads. The segment of a row is chosen
+// among values, not by address: indexing the argument table by a row's segment
+// is a vector load, and its wait would also wait for x. At the sizes of a layer's
+// projections this chain of waits is the bound (kernel us in a replayed graph, with
+// the argument table indexed / this): 2560 rows of 1536, f16 4.72 / 4.20, q4k
+// 4.72 / 3.92; 1536 rows of 2048, q4k 4.52 / 3.88.
+struct LinearTail {
+    const uint16_t* meta[kLinearMaxSegs];
+    float* y[kLinearMaxSegs];
+    const void* w3;
+    uint32_t first3;
+    uint32_t pad;
+};
+
+template <int FMT, int NJ, bool FOUR>
+__global__ __launch_bounds__(256) void k_linear(const float* x, const void* w0, const void* w1, const void* w2,
+                                                uint32_t first1, uint32_t first2, uint32_t total_rows,
+                                                uint32_t rows_per_wave, LinearTail t) {
     const unsigned lane = threadIdx.x & 63;
     const unsigned lq = lane & 31, half = lane >> 5;
+    const unsigned gw = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned r0 = min(gw * rows_per_wave, total_rows - 1);  // a wave past the end repeats the last row
+    const unsigned r1 = min(gw * rows_per_wave + rows_per_wave, total_rows);
+    const uint32_t first3 = FOUR ? t.first3 : ~0u;
     float xr[NJ][8];
-    gemv_load_x<NJ>(a.x, lq, xr);
-    const unsigned gw = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const unsigned r0 = gw * a.rows_per_wave;
-    const unsigned r1 = min(r0 + a.rows_per_wave, a.total_rows);
-    for (unsigned r = r0; r < r1; r += 2) {
+    gemv_load_x<NJ>(x, lq, xr);
+    for (unsigned r = r0;;) {
         const unsigned row = r + half;
-        const bool valid = row < r1;
-        const unsigned gr = valid ? row : r1 - 1;  // clamped: the duplicate's value is discarded
-        int s = 0;
-#pragma unroll
-        for (int i = 1; i < kLinearMaxSegs; i++)
-            if (i < (int)a.n_segs && gr >= a.seg[i].first) s = i;
-        const LinearSegDev& sg = a.seg[s];
-        const unsigned lr = gr - sg.first;
+        const unsigned gr = min(row, r1 - 1);  // clamped: the duplicate's value is discarded
+        const bool s1 = gr >= first1, s2 = gr >= first2, s3 = FOUR && gr >= first3;
+        auto pick = [&](auto a, auto b, auto c, auto d) {
+            auto v = s1 ? b : a;
+            v = s2 ? c : v;
+            if constexpr (FOUR) v = s3 ? d : v;
+            return v;
+        };
+        LinearSegDev sg{};
+        sg.w = pick(w0, w1, w2, t.w3);
+        if constexpr (FMT != kF16) sg.meta = pick(t.meta[0], t.meta[1], t.meta[2], t.meta[3]);
+        const unsigned lr = gr - pick(0u, first1, first2, first3);
         const float v = linear_row<FMT, NJ>(sg, lr, xr, lq);  // the row's value in lane 0 of the half
-        if (valid && lq == 0) sg.y[lr] = v;
+        if (row < r1 && lq == 0) pick(t.y[0], t.y[1], t.y[2], t.y[3])[lr] = v;
+        r += 2;
+        if (r >= r1) return;
     }
 }
 
@@ -82,7 +108,7 @@ unsigned linear_resident_waves() {
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
     if (!cached[dev]) {
         int per_cu = 0, cus = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_linear<FMT, NJ>, 256, 0) != hipSuccess || per_cu < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_linear<FMT, NJ, false>, 256, 0) != hipSuccess || per_cu < 1)
             per_cu = 1;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
         cached[dev] = (unsigned)per_cu * (unsigned)cus * 4;
@@ -95,9 +121,23 @@ int launch_linear(LinearArgs& a, hipStream_t st) {
     const unsigned waves = linear_resident_waves<FMT, NJ>();
     unsigned rpw = 2 * ((a.total_rows + 2 * waves - 1) / (2 * waves));
     if (rpw < 2) rpw = 2;
-    a.rows_per_wave = rpw;
     const unsigned n_waves = (a.total_rows + rpw - 1) / rpw;
-    G4_LAUNCH((k_linear<FMT, NJ>), dim3((n_waves + 3) / 4), dim3(256), 0, st, a);
+    LinearTail t{};
+    uint32_t first[kLinearMaxSegs];
+    for (int i = 0; i < kLinearMaxSegs; i++) {
+        t.meta[i] = a.seg[i].meta;
+        t.y[i] = a.seg[i].y;
+        first[i] = i < (int)a.n_segs ? a.seg[i].first : ~0u;
+    }
+    t.w3 = a.seg[3].w;
+    t.first3 = first[3];
+    const dim3 grid((n_waves + 3) / 4), block(256);
+    if (a.n_segs == 4)
+        G4_LAUNCH((k_linear<FMT, NJ, true>), grid, block, 0, st, a.x, a.seg[0].w, a.seg[1].w, a.seg[2].w, first[1],
+                  first[2], a.total_rows, rpw, t);
+    else
+        G4_LAUNCH((k_linear<FMT, NJ, false>), grid, block, 0, st, a.x, a.seg[0].w, a.seg[1].w, a.seg[2].w, first[1],
+                  first[2], a.total_rows, rpw, t);
     G4_CHECK_LAUNCH("linear");
     return G4_OK;
 }
@@ -280,7 +320,6 @@ __global__ __launch_bounds__(256) void k_linear_prep(LinearArgs a, QkvPrepDev e)
 
 template <int FMT, int NJ>
 int launch_linear_prep(LinearArgs& a, const QkvPrepDev& e, hipStream_t st) {
-    a.rows_per_wave = 2;
     G4_LAUNCH((k_linear_prep<FMT, NJ>), dim3(a.total_rows / kPrepRowsPerWg), dim3(256), 0, st, a, e);
     G4_CHECK_LAUNCH("linearQkvPrep");
     return G4_OK;
