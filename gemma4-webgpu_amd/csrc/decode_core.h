@@ -165,6 +165,18 @@ struct DecodeSmem {
     float l[W][kMaxGroup];
 };
 
+// Eight waves at head_dim 512: the outputs take the place of the score operand,
+// which is read no more when they are published (a barrier apart).
+template <>
+struct DecodeSmem<512, 8> {
+    union {
+        f16x8 q[DecodeDims<512>::NC][64];
+        float o[8][DecodeDims<512>::NO * 4][32];
+    };
+    float m[8][kMaxGroup];
+    float l[8][kMaxGroup];
+};
+
 // Writes 8 consecutive q values (already times scale*log2(e)) of one column as
 // the lane's chunk c of the score operand: hi part in columns 0..7, lo in 8..15.
 template <int HD, int W>
@@ -322,6 +334,96 @@ __device__ __forceinline__ void tile_step(const DecodeSmem<HD, W>& sm, int lane,
     tile_update<HD>(s, g, lo_col, kt0, k1, vreg, m_run, l_run, acc);
 }
 
+// ---- 16-row tiles -------------------------------------------------------------
+//
+// Half of a 32-row tile, for a wave that has 256 registers: at head_dim 512 the
+// accumulators take 128 of them, a tile's K (or V) 64, so after the first tile V
+// is requested when the scores have consumed K and the next K when the outputs
+// have consumed V.
+// The layouts are the 32-row tile's; the output MFMA takes 16 rows
+// (v_mfma_f32_16x16x16_f16: lane (n, g) holds rows 4g .. 4g + 3 of V^T column n
+// and of the probabilities, which is where the scores already lie).
+
+template <int HD, bool kStream>
+__device__ __forceinline__ void load_k_tile16(const char* Kb, uint32_t row_bytes, unsigned last, int n, int g, unsigned kt0,
+                                              f16x8 (&kr)[DecodeDims<HD>::NC]) {
+    const uint32_t off = min(kt0 + n, last) * row_bytes + (uint32_t)g * 16u;
+#pragma unroll
+    for (int c = 0; c < DecodeDims<HD>::NC; c++) kr[c] = ldg_row<kStream, f16x8>(Kb + (off + c * 64u));
+}
+
+template <int HD, bool kStream>
+__device__ __forceinline__ void load_v_tile16(const char* Vb, uint32_t row_bytes, unsigned last, int n, int g, unsigned kt0,
+                                              u32x4 (&vr)[DecodeDims<HD>::NB][4]) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const uint32_t off = min(kt0 + 4 * g + t, last) * row_bytes + (uint32_t)n * 16u;
+#pragma unroll
+        for (int b = 0; b < DecodeDims<HD>::NB; b++) vr[b][t] = ldg_row<kStream, u32x4>(Vb + (off + b * 256u));
+    }
+}
+
+template <int HD, int W>
+__device__ __forceinline__ f32x4 tile_scores16(const DecodeSmem<HD, W>& sm, int lane,
+                                               const f16x8 (&kreg)[DecodeDims<HD>::NC]) {
+    f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < DecodeDims<HD>::NC; c++) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(kreg[c], sm.q[c][lane], s, 0, 0, 0);
+    return s;
+}
+
+// The online softmax of a 16-row tile's scores: updates (m, l) and rescales the
+// accumulators as tile_update does, and returns the probabilities' operand.
+template <int HD>
+__device__ __forceinline__ f16x4 tile_softmax16(const f32x4& s, int g, bool lo_col, unsigned kt0, unsigned k1, float& m_run,
+                                                float& l_run, f32x4 (&acc)[DecodeDims<HD>::NO]) {
+    float sv[4];
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float x = dpp_ror8_add(s[j]);
+        sv[j] = kt0 + g * 4 + j < k1 ? x : -INFINITY;
+        tmax = fmaxf(tmax, sv[j]);
+    }
+    tmax = max_xor16(tmax);
+    tmax = max_xor32(tmax);
+    const float m_new = fmaxf(m_run, tmax);
+    if (__any(m_new > m_run)) {
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
+#pragma unroll
+        for (int i = 0; i < DecodeDims<HD>::NO; i++) acc[i] *= alpha;
+    }
+    m_run = m_new;
+    f16x4 pop;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const float p = __builtin_amdgcn_exp2f(sv[j] - m_new);
+        l_run += p;
+        const f16 hi = (f16)p;
+        pop[j] = lo_col ? (f16)(p - (float)hi) : hi;
+    }
+    return pop;
+}
+
+template <int HD>
+__device__ __forceinline__ void tile_output16(f16x4 pop, const u32x4 (&vreg)[DecodeDims<HD>::NB][4],
+                                              f32x4 (&acc)[DecodeDims<HD>::NO]) {
+#pragma unroll
+    for (int b = 0; b < DecodeDims<HD>::NB; b++) {
+#pragma unroll
+        for (int e2 = 0; e2 < 4; e2++) {
+            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+            const u32x2 lo{perm_lo(vreg[b][0][e2], vreg[b][1][e2]), perm_lo(vreg[b][2][e2], vreg[b][3][e2])};
+            const u32x2 hi{perm_hi(vreg[b][0][e2], vreg[b][1][e2]), perm_hi(vreg[b][2][e2], vreg[b][3][e2])};
+            acc[b * 8 + 2 * e2] =
+                __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, lo), pop, acc[b * 8 + 2 * e2], 0, 0, 0);
+            acc[b * 8 + 2 * e2 + 1] =
+                __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(f16x4, hi), pop, acc[b * 8 + 2 * e2 + 1], 0, 0, 0);
+        }
+    }
+}
+
 // Publishes a wave's final state to workgroup memory (sums over the 4 lane
 // groups, hi + lo columns added).
 template <int HD, int W>
@@ -359,7 +461,9 @@ __device__ __forceinline__ void wave_publish(DecodeSmem<HD, W>& sm, int wave, in
 // `extra_m` (optional, per head, log2 units) with `extra_v` (one f16 row shared
 // by the heads) adds a further state holding a single row of weight 1: the
 // current token's row when it was not part of the tile loop.
-template <int HD, int W>
+// LW: the combine reads the first LW waves' states (of the W that could be
+// published; the thread mapping is W's).
+template <int HD, int W, int LW = W>
 __device__ __forceinline__ void wg_combine_write(const DecodeSmem<HD, W>& sm, unsigned G, bool final_out, float* out,
                                                  float* part_o, float* part_ml, const float* extra_m = nullptr,
                                                  const f16* extra_v = nullptr, int t = threadIdx.x) {
@@ -371,17 +475,17 @@ __device__ __forceinline__ void wg_combine_write(const DecodeSmem<HD, W>& sm, un
     const int h = lane32 & 7;
     const int gg = lane32 >> 3;
     if ((unsigned)h >= G) return;
-    float mw[W], M = -INFINITY;
+    float mw[LW], M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < W; w++) {
+    for (int w = 0; w < LW; w++) {
         mw[w] = sm.m[w][h];
         M = fmaxf(M, mw[w]);
     }
     const float me = extra_m ? extra_m[h] : -INFINITY;
     M = fmaxf(M, me);
-    float L = 0.0f, sc[W];
+    float L = 0.0f, sc[LW];
 #pragma unroll
-    for (int w = 0; w < W; w++) {
+    for (int w = 0; w < LW; w++) {
         sc[w] = __builtin_amdgcn_exp2f(mw[w] - M);
         L += sm.l[w][h] * sc[w];
     }
@@ -402,7 +506,7 @@ __device__ __forceinline__ void wg_combine_write(const DecodeSmem<HD, W>& sm, un
             const int sl = (b * 8 + e0 + e) * 4 + j;
             float v = 0.0f;
 #pragma unroll
-            for (int w = 0; w < W; w++) v += sm.o[w][sl][lane32] * sc[w];
+            for (int w = 0; w < LW; w++) v += sm.o[w][sl][lane32] * sc[w];
             if (extra_m) v += (float)extra_v[d0 + e] * se;
             o[e] = final_out ? v * inv_l : v;
         }

@@ -71,11 +71,14 @@ struct StepSmem {
     float mnew[kMaxGroup];    // current row's scores (log2 units)
 };
 
-// W waves per workgroup. head_dim 256: two waves per SIMD (two 4-wave
-// workgroups or one 8-wave workgroup per CU), enough rows in flight to cover
-// the HBM latency with one 32-row tile per wave. head_dim 512: one 4-wave
-// workgroup per CU at one wave per SIMD (a 32-row tile is 64 KB of K and V,
-// the accumulators take 128 registers more).
+// W waves per workgroup, two waves per SIMD (two 4-wave workgroups or one 8-wave
+// workgroup per CU), enough rows in flight to cover the HBM latency with one
+// tile per wave: 32 rows at head_dim 256, 16 at 512, where the accumulators take
+// 128 of a wave's 256 registers. At 512 one 4-wave workgroup per CU with 32-row
+// tiles at one wave per SIMD has nothing to run while its tile's loads are out,
+// and two query heads per wave in the prologue (us per step of one layer, that
+// form / this: 1023 rows 12.9 / 10.8, 4096 13.2 / 12.5, 32768 24.6 / 24.2, 100000
+// 45.8 / 44.1; a token of both head_dims with shared caches at 32768 70.4 / 64.2).
 //
 // The arguments are scalars and pointers (not one struct) so that they are
 // preloaded into SGPRs at wave start (the file is compiled with kernarg
@@ -122,8 +125,9 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
     const unsigned nkeys = k1t - k0;
     const unsigned last = nkeys ? k1t - 1 : k0;  // loads are clamped to it (k0 < key_end: in the cache)
 
-    constexpr unsigned kStride = W * kTileKeys;
-    unsigned t0 = (unsigned)wave * kTileKeys;
+    constexpr unsigned kRows = HD == 512 ? 16 : kTileKeys;  // rows of a wave's tile
+    constexpr unsigned kStride = W * kRows;
+    unsigned t0 = (unsigned)wave * kRows;
     float m_run = -INFINITY, l_run = 0.0f;
     f32x4 acc[D::NO];
 #pragma unroll
@@ -185,15 +189,17 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
         const uint32_t row_bytes = NKH * HD * 2u;
         const char* Kb = reinterpret_cast<const char*>(ent.k_cache + (uint64_t)kvh * HD);
         const char* Vb = reinterpret_cast<const char*>(ent.v_cache + (uint64_t)kvh * HD);
-        f16x8 kreg[2][D::NC];
-        u32x4 vreg[D::NB][8];
-        auto load_tile = [&] {  // the tile at t0
-            load_k_tile<HD, !KEEP>(Kb, row_bytes, last, n, g, k0 + t0, kreg);
-            load_v_tile<HD, !KEEP>(Vb, row_bytes, last, n, g, k0 + t0, vreg);
+        f16x8 kreg[kRows / 16][D::NC];
+        u32x4 vreg[D::NB][kRows / 4];
+        auto load_tile = [&] {  // the tile at t0 (of a 16-row tile, K alone)
+            if constexpr (kRows == 16) {
+                load_k_tile16<HD, !KEEP>(Kb, row_bytes, last, n, g, k0 + t0, kreg[0]);
+            } else {
+                load_k_tile<HD, !KEEP>(Kb, row_bytes, last, n, g, k0 + t0, kreg);
+                load_v_tile<HD, !KEEP>(Vb, row_bytes, last, n, g, k0 + t0, vreg);
+            }
         };
-        if constexpr (kTile) {
-            load_tile();
-        }
+        if constexpr (kTile) load_tile();
         __builtin_amdgcn_sched_barrier(0);  // keep every request above ahead of the arithmetic below
 
         // ---- q heads straight into the score operand; the current row's k and v ----
@@ -266,10 +272,22 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
 
         // ---- tiles ----
         if constexpr (kTile) {  // the first tile was requested above; the loop requests its own
-            tile_step<HD>(sm.dec, lane, g, lo_col, k0 + t0, k1t, kreg, vreg, m_run, l_run, acc);
+            auto use_tile = [&] {
+                if constexpr (kRows == 16) {
+                    const f32x4 sc = tile_scores16<HD>(sm.dec, lane, kreg[0]);
+                    __builtin_amdgcn_sched_barrier(0);  // V into K's registers
+                    load_v_tile16<HD, !KEEP>(Vb, row_bytes, last, n, g, k0 + t0, vreg);
+                    const f16x4 pop = tile_softmax16<HD>(sc, g, lo_col, k0 + t0, k1t, m_run, l_run, acc);
+                    tile_output16<HD>(pop, vreg, acc);
+                    __builtin_amdgcn_sched_barrier(0);  // the next K into V's
+                } else {
+                    tile_step<HD>(sm.dec, lane, g, lo_col, k0 + t0, k1t, kreg, vreg, m_run, l_run, acc);
+                }
+            };
+            use_tile();
             for (t0 += kStride; t0 < nkeys; t0 += kStride) {
                 load_tile();
-                tile_step<HD>(sm.dec, lane, g, lo_col, k0 + t0, k1t, kreg, vreg, m_run, l_run, acc);
+                use_tile();
             }
         }
     };
@@ -277,21 +295,37 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
         body(std::true_type{});
     else
         body(std::false_type{});
-    wave_publish<HD>(sm.dec, wave, n, g, m_run, l_run, acc);
+    // The waves that have rows are the first ones. At head_dim 512 a part that keeps 2, 4 or 6 waves busy
+    // publishes and combines those alone (the states of the others weigh 0): a wave's outputs are 16 KB
+    // of LDS written and read. One layer at position 1023 / 4096 (us with the merge): 12.3 / 13.7 with all
+    // eight states, 10.8 / 12.5 so. At head_dim 256 (half the outputs) it gave nothing.
+    constexpr bool kFew = HD == 512;
+    const unsigned used = kFew ? min((unsigned)W, max(2u, ((nkeys + kRows - 1) / kRows + 1) & ~1u)) : (unsigned)W;
+    if constexpr (HD == 512) __syncthreads();  // every wave has read its last score operand
+    if (!kFew || (unsigned)wave < used) wave_publish<HD>(sm.dec, wave, n, g, m_run, l_run, acc);
     __syncthreads();
 
     const float* em = has_new ? sm.mnew : nullptr;
     const f16* ev = reinterpret_cast<const f16*>(sm.vnew);
-    if (ent.n_parts == 1) {
-        wg_combine_write<HD>(sm.dec, G, true, ent.out + (uint64_t)kvh * G * HD, nullptr, nullptr, em, ev);
-        return;
+    auto combine = [&](auto waves) __attribute__((always_inline)) {
+        constexpr int LW = decltype(waves)::value;
+        if (ent.n_parts == 1) {
+            wg_combine_write<HD, W, LW>(sm.dec, G, true, ent.out + (uint64_t)kvh * G * HD, nullptr, nullptr, em, ev);
+            return;
+        }
+        const uint64_t rec = ((uint64_t)wk.part * NKH + kvh) * G;
+        wg_combine_write<HD, W, LW>(sm.dec, G, false, nullptr, a.part_o + rec * HD, a.part_ml + rec * 2, em, ev);
+    };
+    if constexpr (kFew) {
+        if (used == 2) return combine(std::integral_constant<int, 2>{});
+        if (used == 4) return combine(std::integral_constant<int, 4>{});
+        if (used == 6) return combine(std::integral_constant<int, 6>{});
     }
-    const uint64_t rec = ((uint64_t)wk.part * NKH + kvh) * G;
-    wg_combine_write<HD>(sm.dec, G, false, nullptr, a.part_o + rec * HD, a.part_ml + rec * 2, em, ev);
+    combine(std::integral_constant<int, W>{});
 }
 
 template <int W, int HD, bool KEEP>
-__global__ __launch_bounds__(64 * W, HD == 256 ? 8 / W : 1) void k_attn_step(
+__global__ __launch_bounds__(64 * W, 8 / W) void k_attn_step(
     const StepWorkDev* __restrict__ work, float* part_ml, float* part_o, uint32_t num_kv_heads, uint32_t group,
     uint32_t adv) {
     __shared__ StepSmem<W, HD> sm;
@@ -300,24 +334,24 @@ __global__ __launch_bounds__(64 * W, HD == 256 ? 8 / W : 1) void k_attn_step(
 
 // Two plans of one token in one launch (E2B's two head_dim groups): the
 // head_dim-512 plan's workgroups first, one per CU, then the head_dim-256
-// plan's, in 4-wave workgroups of the same size, which take the CUs the first
+// plan's, in 8-wave workgroups of the same size, which take the CUs the first
 // ones leave as they finish. Grid: (wgs_a + wgs_b) x the larger kv-head count.
 union StepPairSmem {
-    StepSmem<4, 512> a;
-    StepSmem<4, 256> b;
+    StepSmem<8, 512> a;
+    StepSmem<8, 256> b;
 };
 
 template <bool KEEP>
-__global__ __launch_bounds__(256, 1) void k_attn_step_pair(
+__global__ __launch_bounds__(512, 1) void k_attn_step_pair(
     const StepWorkDev* __restrict__ work_a, float* ml_a, float* o_a, uint32_t nkh_a, uint32_t group_a, uint32_t adv_a,
     uint32_t wgs_a, const StepWorkDev* __restrict__ work_b, float* ml_b, float* o_b, uint32_t nkh_b, uint32_t group_b,
     uint32_t adv_b) {
     __shared__ StepPairSmem sm;
     const unsigned x = blockIdx.x, y = blockIdx.y;
     if (x < wgs_a) {  // uniform
-        if (y < nkh_a) attn_step_body<4, 512, KEEP>(work_a, ml_a, o_a, nkh_a, group_a, adv_a, x, y, sm.a);
+        if (y < nkh_a) attn_step_body<8, 512, KEEP>(work_a, ml_a, o_a, nkh_a, group_a, adv_a, x, y, sm.a);
     } else if (y < nkh_b) {
-        attn_step_body<4, 256, KEEP>(work_b, ml_b, o_b, nkh_b, group_b, adv_b, x - wgs_a, y, sm.b);
+        attn_step_body<8, 256, KEEP>(work_b, ml_b, o_b, nkh_b, group_b, adv_b, x - wgs_a, y, sm.b);
     }
 }
 
@@ -512,7 +546,7 @@ static int launch_attention(const g4_decode_plan* plan, void* stream, hipEvent_t
             G4_LAUNCH(kernel, grid, dim3(threads), 0, st, a.work, a.part_ml, a.part_o, a.num_kv_heads, a.group, adv);
     };
     if (r.head_dim == 512)
-        r.keep_rows ? launch(k_attn_step<4, 512, true>, 256) : launch(k_attn_step<4, 512, false>, 256);
+        r.keep_rows ? launch(k_attn_step<8, 512, true>, 512) : launch(k_attn_step<8, 512, false>, 512);
     else if (r.waves == 8)
         r.keep_rows ? launch(k_attn_step<8, 256, true>, 512) : launch(k_attn_step<8, 256, false>, 512);
     else
@@ -545,11 +579,11 @@ static int launch_attention_pair(const g4_decode_plan* plan_1, const g4_decode_p
     hipStream_t st = as_stream(stream);
     auto launch = [&](auto kernel) {
         if (start || stop)
-            hipExtLaunchKernelGGL(kernel, grid, dim3(256), 0, st, start, stop, 0, wa, ml(a), po(a),
+            hipExtLaunchKernelGGL(kernel, grid, dim3(512), 0, st, start, stop, 0, wa, ml(a), po(a),
                                   (uint32_t)a.num_kv_heads, (uint32_t)a.group, a.adv, (uint32_t)a.n_wgs, wb, ml(b),
                                   po(b), (uint32_t)b.num_kv_heads, (uint32_t)b.group, b.adv);
         else
-            G4_LAUNCH(kernel, grid, dim3(256), 0, st, wa, ml(a), po(a), (uint32_t)a.num_kv_heads, (uint32_t)a.group,
+            G4_LAUNCH(kernel, grid, dim3(512), 0, st, wa, ml(a), po(a), (uint32_t)a.num_kv_heads, (uint32_t)a.group,
                       a.adv, (uint32_t)a.n_wgs, wb, ml(b), po(b), (uint32_t)b.num_kv_heads, (uint32_t)b.group, b.adv);
     };
     a.keep_rows || b.keep_rows ? launch(k_attn_step_pair<true>) : launch(k_attn_step_pair<false>);
@@ -630,14 +664,7 @@ int g4_attn_step_run_merge(const g4_decode_plan* plan, void* stream) {
     int rc = step_plan(plan, &r);
     if (rc) return rc;
     if (!r.n_merge) return G4_OK;
-    DecodeArgs m = {};
-    m.table = reinterpret_cast<const DecodeEntryDev*>(r.tables + r.off_merge);
-    m.n_entries = r.n_merge;
-    m.num_kv_heads = r.num_kv_heads;
-    m.group = r.group;
-    m.part_ml = reinterpret_cast<float*>(r.part_ml);
-    m.part_o = reinterpret_cast<float*>(r.part_ml + step_part_o_offset(r.num_kv_heads, r.group));
-    return launch_decode_merge(m, r.n_merge, r.max_parts, as_stream(stream), r.head_dim);
+    return launch_decode_merge(merge_args(r), r.n_merge, r.max_parts, as_stream(stream), r.head_dim);
 }
 
 int g4_attn_step_run_out(const g4_decode_plan* plan, const g4_linear_seg* o_proj, uint32_t n_segs, void* stream) {

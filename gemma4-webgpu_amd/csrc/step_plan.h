@@ -376,11 +376,11 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
     // 190.9 / 199.6 / 197.8. A second workgroup per CU starts behind the first
     // and is served after it, which only pays off when the per-wave rounds
     // are many; grids between one and two per CU are slower than both (CUs
-    // with two workgroups finish last). head_dim 512 has one form: one 4-wave
+    // with two workgroups finish last). head_dim 512 has one form: one 8-wave
     // workgroup per CU.
     if (cus < 1) cus = 1;
     const bool small = T <= (uint64_t)kStepOneWgTiles * (cus / num_kv_heads);
-    const uint32_t waves = head_dim == 512 ? 4u
+    const uint32_t waves = head_dim == 512 ? 8u
                            : tune.waves == 4 || tune.waves == 8 ? (uint32_t)tune.waves
                                                                  : (small ? 8u : 4u);
     const uint64_t per_cu = head_dim == 512 ? 1u
@@ -395,7 +395,9 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
     // two tiles per workgroup instead of one cost no extra tile round and halve
     // the partial records. Measured on one local layer (16 tiles, us per step
     // with the merge): 16 workgroups 10.82, 8 workgroups 10.20, 4 workgroups 10.47.
-    if (waves == 8 && tune.max_wgs <= 0 && tpw < 2 && max_tiles >= 2) tpw = 2;
+    // At head_dim 512 a tile already keeps two waves busy, and one per workgroup is
+    // the faster split (one layer at 1023: 12.3 against 12.8).
+    if (waves == 8 && head_dim == 256 && tune.max_wgs <= 0 && tpw < 2 && max_tiles >= 2) tpw = 2;
 
     // Sizes: work items (tpw tiles each, balanced within an entry), merge
     // entries (entries with partial records: the merge grid covers them alone).
@@ -468,48 +470,59 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
     // Work items, in the order of the workgroups that take them: entry by entry,
     // part by part. Workgroup w runs on XCD w % 8, each with its own L2, so when
     // entries share cache rows the items of one part of a group (the same rows,
-    // different queries) take consecutive workgroups of one XCD: its L2 then reads
-    // those rows once for most of them. Measured on a token of E2B's real shapes
-    // (us, one state / three in turn): position 32768 81.0 / 85.9 entry by entry
-    // with streaming loads, 78.2 in this order, 70.4 / 76.6 in this order with
-    // ordinary loads; 16384 56.0 -> 41.6; 8192 37.3 -> 30.6; 2048 23.0 -> 21.1.
-    size_t at = 0, xcd = 0;
-    auto next_item = [&]() -> StepWorkDev& {
-        StepWorkDev& w = work[at];
-        if (!shared) {
-            at++;
-        } else if ((at += kXcds) >= n_work) {
-            at = ++xcd;
-        }
-        return w;
-    };
-    for (uint32_t i = 0; i < n_entries; i++) {
-        if (shared && ph.kv_first[i] != i) continue;  // placed with its group
-        // Part j covers tiles [j ne / we, (j + 1) ne / we): the bounds advance by
-        // ne / we and carry the remainder, with no division per part.
-        const uint64_t ne = tiles[i], we = ph.tab[i].n_parts;
-        const uint64_t step = ne / we, rem = ne % we;
-        uint64_t te = 0, acc = 0;
-        for (uint64_t j = 0; j < we; j++) {
-            const uint64_t tb = te;
-            te += step;
-            acc += rem;
-            if (acc >= we) {
-                acc -= we;
-                te++;
-            }
-            const uint64_t rb = key_begin[i] + tb * kTileKeys;
-            const uint64_t re = key_begin[i] + te * kTileKeys;
-            for (uint32_t m = i; m != ~0u; m = shared ? ph.kv_next[m] : ~0u) {  // the same rows, hence the same parts
-                StepWorkDev& w = next_item();
-                w.ent = ph.tab[m];
-                w.row_begin = (uint32_t)rb;
-                w.row_end = (uint32_t)(re < w.ent.key_end ? re : w.ent.key_end);
-                w.part = we > 1 ? ph.part_base[m] + (uint32_t)j : 0u;
-                w.entry = m;
-            }
-        }
+    // different queries) go to one XCD, whose L2 then reads those rows once for
+    // all of them; the parts go to the XCD with the most workgroups left (groups
+    // first), which spreads the distinct rows evenly too. Measured on a token of
+    // E2B's real shapes (us, two states in turn): position 32768 80.9 entry by entry
+    // with streaming loads, 64.1 so with ordinary ones (73.7 so with streaming ones);
+    // 16384 56.0 / 37.1, 8192 37.3 / 27.9, 2048 23.0 / 19.1. With the groups' parts on
+    // consecutive XCDs, not spread, 32768 took 69.0: the entries without a group then
+    // sat on two XCDs, whose share of the memory bandwidth bounded the launch.
+    uint64_t next[kXcds], left[kXcds];  // an XCD's next workgroup, and how many it has left
+    for (uint64_t c = 0; c < kXcds; c++) {
+        next[c] = c;
+        left[c] = n_work > c ? (n_work - c + kXcds - 1) / kXcds : 0;
     }
+    uint64_t at = 0;
+    for (int singles = 0; singles < (shared ? 2 : 1); singles++)
+        for (uint32_t i = 0; i < n_entries; i++) {
+            // A group is placed with its first entry, in the first round; entries on their own in the second.
+            if (shared && (ph.kv_first[i] != i || (ph.kv_next[i] == ~0u) != (singles == 1))) continue;
+            // Part j covers tiles [j ne / we, (j + 1) ne / we): the bounds advance by
+            // ne / we and carry the remainder, with no division per part.
+            const uint64_t ne = tiles[i], we = ph.tab[i].n_parts;
+            const uint64_t step = ne / we, rem = ne % we;
+            uint64_t te = 0, acc = 0;
+            for (uint64_t j = 0; j < we; j++) {
+                const uint64_t tb = te;
+                te += step;
+                acc += rem;
+                if (acc >= we) {
+                    acc -= we;
+                    te++;
+                }
+                const uint64_t rb = key_begin[i] + tb * kTileKeys;
+                const uint64_t re = key_begin[i] + te * kTileKeys;
+                uint64_t xcd = 0;
+                if (shared)
+                    for (uint64_t c = 1; c < kXcds; c++)
+                        if (left[c] > left[xcd]) xcd = c;
+                for (uint32_t m = i; m != ~0u; m = shared ? ph.kv_next[m] : ~0u) {  // the same rows, so the same parts
+                    if (shared) {
+                        while (!left[xcd]) xcd = (xcd + 1) % kXcds;
+                        at = next[xcd];
+                        next[xcd] += kXcds;
+                        left[xcd]--;
+                    }
+                    StepWorkDev& w = work[at++];
+                    w.ent = ph.tab[m];
+                    w.row_begin = (uint32_t)rb;
+                    w.row_end = (uint32_t)(re < w.ent.key_end ? re : w.ent.key_end);
+                    w.part = we > 1 ? ph.part_base[m] + (uint32_t)j : 0u;
+                    w.entry = m;
+                }
+            }
+        }
     ph.keep_rows = shared;
     ph.waves = waves;
     ph.n_wgs = (uint32_t)n_work;
