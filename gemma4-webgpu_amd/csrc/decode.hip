@@ -18,6 +18,7 @@
 
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "decode_core.h"
@@ -142,15 +143,26 @@ __device__ __forceinline__ DecodeEntryDev merge_entry(const DecodeEntryDev* tabl
     return e;
 }
 
-// One workgroup (entry bx, query head by of its kv head, column chunk bz) of k_decode_merge.
+// The entry of token bx of a table of token runs: 2^shift tokens per entry, of
+// which the first `pad` exist; a token's attnOut lies `stride` floats after the
+// token before, its records n_splits after. Absent tokens come back without records.
+__device__ __forceinline__ DecodeEntryDev merge_token(const DecodeEntryDev* __restrict__ table, uint32_t shift,
+                                                      uint32_t stride, unsigned bx) {
+    DecodeEntryDev e = table[bx >> shift];
+    const unsigned tk = bx & ((1u << shift) - 1u);
+    e.out += (uint64_t)tk * stride;
+    e.split_base += tk * e.n_splits;
+    if (tk >= e.pad) e.n_splits = 0;
+    return e;
+}
+
+// One workgroup (an entry, query head by of its kv head, column chunk bz) of k_decode_merge.
 template <int HD>
-__device__ __forceinline__ void merge_body(const DecodeEntryDev* __restrict__ table, float* one_out,
-                                           uint32_t one_split_base, uint32_t one_splits, float* part_ml,
-                                           float* part_o, uint32_t num_kv_heads, uint32_t group, uint32_t n_chunks,
-                                           unsigned bx, unsigned by, unsigned bz) {
+__device__ __forceinline__ void merge_body(const DecodeEntryDev& ent, float* part_ml, float* part_o,
+                                           uint32_t num_kv_heads, uint32_t group, uint32_t n_chunks, unsigned by,
+                                           unsigned bz) {
     __shared__ f32x4 part[kMergeThreads];
     __shared__ float gm[kMergeThreads], gl[kMergeThreads];  // per group: running max, rescaled l
-    const DecodeEntryDev ent = merge_entry(table, one_out, one_split_base, one_splits, bx);
     DecodeArgs a{};
     a.num_kv_heads = num_kv_heads;
     a.group = group;
@@ -225,8 +237,21 @@ __global__ __launch_bounds__(kMergeThreads) void k_decode_merge(const DecodeEntr
                                                                 uint32_t one_split_base, uint32_t one_splits,
                                                                 float* part_ml, float* part_o, uint32_t num_kv_heads,
                                                                 uint32_t group, uint32_t n_chunks) {
-    merge_body<HD>(table, one_out, one_split_base, one_splits, part_ml, part_o, num_kv_heads, group, n_chunks,
-                   blockIdx.x, blockIdx.y, blockIdx.z);
+    merge_body<HD>(merge_entry(table, one_out, one_split_base, one_splits, blockIdx.x), part_ml, part_o, num_kv_heads,
+                   group, n_chunks, blockIdx.y, blockIdx.z);
+}
+
+// The merges of prefill tokens: a table entry is a query tile cut into key parts,
+// and a workgroup derives its token's records and attnOut from it. (With an entry
+// per token the host builds and uploads 56 bytes a token: a prompt of 1000 tokens
+// over two layers, planned in the call, took 56.3 us with that and takes 49.2 so.)
+template <int HD>
+__global__ __launch_bounds__(kMergeThreads) void k_token_merge(const DecodeEntryDev* __restrict__ table, uint32_t shift,
+                                                               uint32_t stride, float* part_ml, float* part_o,
+                                                               uint32_t num_kv_heads, uint32_t group,
+                                                               uint32_t n_chunks) {
+    merge_body<HD>(merge_token(table, shift, stride, blockIdx.x), part_ml, part_o, num_kv_heads, group, n_chunks,
+                   blockIdx.y, blockIdx.z);
 }
 
 // The same merge for entries of at most kSmallMergeSplits records: one
@@ -282,12 +307,9 @@ __device__ __forceinline__ void merge_small_fold(const f32x4 (&v)[NS][COLS / 4],
 // NS: the launch's largest split count rounded up to 2, 4 or 8 (records past an entry's own count
 // are not loaded).
 template <int HD, int COLS, int NS>
-__device__ __forceinline__ void merge_small_body(const DecodeEntryDev* __restrict__ table, float* one_out,
-                                                 uint32_t one_split_base, uint32_t one_splits, float* part_ml,
-                                                 float* part_o, uint32_t num_kv_heads, uint32_t group, unsigned bx,
-                                                 unsigned by) {
+__device__ __forceinline__ void merge_small_body(const DecodeEntryDev& ent, float* part_ml, float* part_o,
+                                                 uint32_t num_kv_heads, uint32_t group, unsigned by) {
     constexpr unsigned TPH = HD / COLS;  // threads per query head
-    const DecodeEntryDev ent = merge_entry(table, one_out, one_split_base, one_splits, bx);
     const unsigned ns = ent.n_splits;
     if (ns <= 1) return;
     const unsigned G = group, kvh = by;
@@ -311,8 +333,17 @@ __global__ __launch_bounds__(kMergeThreads) void k_decode_merge_small(const Deco
                                                                       uint32_t one_splits, float* part_ml,
                                                                       float* part_o, uint32_t num_kv_heads,
                                                                       uint32_t group) {
-    merge_small_body<HD, COLS, NS>(table, one_out, one_split_base, one_splits, part_ml, part_o, num_kv_heads, group,
-                                   blockIdx.x, blockIdx.y);
+    merge_small_body<HD, COLS, NS>(merge_entry(table, one_out, one_split_base, one_splits, blockIdx.x), part_ml, part_o,
+                                   num_kv_heads, group, blockIdx.y);
+}
+
+template <int HD, int COLS, int NS>
+__global__ __launch_bounds__(kMergeThreads) void k_token_merge_small(const DecodeEntryDev* __restrict__ table,
+                                                                     uint32_t shift, uint32_t stride, float* part_ml,
+                                                                     float* part_o, uint32_t num_kv_heads,
+                                                                     uint32_t group) {
+    merge_small_body<HD, COLS, NS>(merge_token(table, shift, stride, blockIdx.x), part_ml, part_o, num_kv_heads, group,
+                                   blockIdx.y);
 }
 
 // The merges of two step plans of one token in one launch (E2B's head_dim-512
@@ -330,49 +361,55 @@ __global__ __launch_bounds__(kMergeThreads) void k_decode_merge_pair(
     if (x < n_a) {  // uniform
         const unsigned e = x % ents_a;
         x /= ents_a;
-        merge_body<512>(table_a, nullptr, 0, 0, ml_a, o_a, nkh_a, group_a, chunks_a, e, x % heads_a, x / heads_a);
+        merge_body<512>(table_a[e], ml_a, o_a, nkh_a, group_a, chunks_a, x % heads_a, x / heads_a);
     } else {
         x -= n_a;
-        merge_small_body<256, COLS, NS>(table_b, nullptr, 0, 0, ml_b, o_b, nkh_b, group_b, x % ents_b, x / ents_b);
+        merge_small_body<256, COLS, NS>(table_b[x % ents_b], ml_b, o_b, nkh_b, group_b, x / ents_b);
     }
 }
 
 #define MERGE_KARGS                                                                                               \
     a.table, a.one.out, a.one.split_base, a.one.n_splits, a.part_ml, a.part_o, a.num_kv_heads, a.group
 
+// One round trip of k_decode_merge covers kMergeBatch * P = kMergeBatch * 4 * kMergeThreads / HD records per chunk.
+template <int HD>
+unsigned merge_chunks(unsigned max_splits) {
+    constexpr unsigned kRecsPerChunk = kMergeBatch * 4 * kMergeThreads / HD;
+    unsigned chunks = 1;
+    while (chunks < kMaxMergeChunks && max_splits > kRecsPerChunk * chunks) chunks *= 2;
+    return chunks;
+}
+
+// Calls f with the record count of the small form (2, 4 or 8) as a constant.
+template <typename F>
+void with_small_splits(unsigned max_splits, F f) {
+    if (max_splits <= 2)
+        f(std::integral_constant<int, 2>{});
+    else if (max_splits <= 4)
+        f(std::integral_constant<int, 4>{});
+    else
+        f(std::integral_constant<int, 8>{});
+}
+
 template <int HD>
 int launch_decode_merge_hd(const DecodeArgs& a, unsigned n_entries, unsigned max_splits, hipStream_t st) {
+    const dim3 block(kMergeThreads);
     if (max_splits <= kSmallMergeSplits && (a.group == 8 || a.group == 4)) {
         const dim3 grid(n_entries, a.num_kv_heads);
-        const dim3 block(kMergeThreads);
-        if (a.group == 8) {
-            constexpr int C = HD * 8 / 256;
-            if (max_splits <= 2)
-                G4_LAUNCH((k_decode_merge_small<HD, C, 2>), grid, block, 0, st, MERGE_KARGS);
-            else if (max_splits <= 4)
-                G4_LAUNCH((k_decode_merge_small<HD, C, 4>), grid, block, 0, st, MERGE_KARGS);
+        with_small_splits(max_splits, [&](auto ns) {
+            constexpr int NS = decltype(ns)::value;
+            if (a.group == 8)
+                G4_LAUNCH((k_decode_merge_small<HD, HD * 8 / 256, NS>), grid, block, 0, st, MERGE_KARGS);
             else
-                G4_LAUNCH((k_decode_merge_small<HD, C, 8>), grid, block, 0, st, MERGE_KARGS);
-        } else {
-            constexpr int C = HD * 4 / 256;
-            if (max_splits <= 2)
-                G4_LAUNCH((k_decode_merge_small<HD, C, 2>), grid, block, 0, st, MERGE_KARGS);
-            else if (max_splits <= 4)
-                G4_LAUNCH((k_decode_merge_small<HD, C, 4>), grid, block, 0, st, MERGE_KARGS);
-            else
-                G4_LAUNCH((k_decode_merge_small<HD, C, 8>), grid, block, 0, st, MERGE_KARGS);
-        }
+                G4_LAUNCH((k_decode_merge_small<HD, HD * 4 / 256, NS>), grid, block, 0, st, MERGE_KARGS);
+        });
         G4_CHECK_LAUNCH("attnDecode merge");
         return G4_OK;
     }
     if (max_splits > (unsigned)kMaxMergeSplits)
         return fail(G4_EINVAL, "attnDecode merge: %u splits (max %d)", max_splits, kMaxMergeSplits);
-    // one round trip covers kMergeBatch * P = kMergeBatch * 4 * kMergeThreads / HD records per chunk
-    constexpr unsigned kRecsPerChunk = kMergeBatch * 4 * kMergeThreads / HD;
-    unsigned chunks = 1;
-    while (chunks < kMaxMergeChunks && max_splits > kRecsPerChunk * chunks) chunks *= 2;
-    G4_LAUNCH(k_decode_merge<HD>, dim3(n_entries, a.num_kv_heads * a.group, chunks), dim3(kMergeThreads), 0,
-                       st, MERGE_KARGS, chunks);
+    const unsigned chunks = merge_chunks<HD>(max_splits);
+    G4_LAUNCH(k_decode_merge<HD>, dim3(n_entries, a.num_kv_heads * a.group, chunks), block, 0, st, MERGE_KARGS, chunks);
     G4_CHECK_LAUNCH("attnDecode merge");
     return G4_OK;
 }
@@ -383,9 +420,7 @@ int launch_decode_merge_pair(const DecodeArgs& a, unsigned n_a, unsigned max_a, 
                              unsigned max_b, hipStream_t st) {
     if (!n_a || max_a <= kSmallMergeSplits || max_a > (unsigned)kMaxMergeSplits) return 1;
     if (!n_b || max_b <= 1 || max_b > kSmallMergeSplits || (b.group != 8 && b.group != 4)) return 1;
-    constexpr unsigned kRecsPerChunk = kMergeBatch * 4 * kMergeThreads / 512;  // as launch_decode_merge_hd<512>
-    unsigned chunks = 1;
-    while (chunks < kMaxMergeChunks && max_a > kRecsPerChunk * chunks) chunks *= 2;
+    const unsigned chunks = merge_chunks<512>(max_a);
     const uint64_t wgs = (uint64_t)n_a * a.num_kv_heads * a.group * chunks + (uint64_t)n_b * b.num_kv_heads;
     if (wgs > 0x7fffffffu) return 1;
     const dim3 grid((uint32_t)wgs), block(kMergeThreads);
@@ -416,6 +451,40 @@ int launch_decode_merge(const DecodeArgs& a, unsigned n_entries, unsigned max_sp
     if (!n_entries || max_splits <= 1) return G4_OK;
     if (head_dim == 512) return launch_decode_merge_hd<512>(a, n_entries, max_splits, st);
     return launch_decode_merge_hd<256>(a, n_entries, max_splits, st);
+}
+
+template <int HD>
+int launch_token_merge_hd(const DecodeArgs& a, unsigned tiles, unsigned shift, unsigned max_splits, hipStream_t st) {
+    const uint64_t tokens = (uint64_t)tiles << shift;
+    const uint32_t stride = a.num_kv_heads * a.group * HD;
+    if (tokens > 0x7fffffffu || max_splits > (unsigned)kMaxMergeSplits)
+        return fail(G4_EINVAL, "attnPrefill merge: %u tiles of %u parts", tiles, max_splits);
+    const dim3 block(kMergeThreads);
+    if (max_splits <= kSmallMergeSplits && (a.group == 8 || a.group == 4)) {
+        const dim3 grid((unsigned)tokens, a.num_kv_heads);
+        with_small_splits(max_splits, [&](auto ns) {
+            constexpr int NS = decltype(ns)::value;
+            if (a.group == 8)
+                G4_LAUNCH((k_token_merge_small<HD, HD * 8 / 256, NS>), grid, block, 0, st, a.table, shift, stride,
+                          a.part_ml, a.part_o, a.num_kv_heads, a.group);
+            else
+                G4_LAUNCH((k_token_merge_small<HD, HD * 4 / 256, NS>), grid, block, 0, st, a.table, shift, stride,
+                          a.part_ml, a.part_o, a.num_kv_heads, a.group);
+        });
+    } else {
+        const unsigned chunks = merge_chunks<HD>(max_splits);
+        G4_LAUNCH(k_token_merge<HD>, dim3((unsigned)tokens, a.num_kv_heads * a.group, chunks), block, 0, st, a.table,
+                  shift, stride, a.part_ml, a.part_o, a.num_kv_heads, a.group, chunks);
+    }
+    G4_CHECK_LAUNCH("attnPrefill merge");
+    return G4_OK;
+}
+
+int launch_token_merge(const DecodeArgs& a, unsigned tiles, unsigned shift, unsigned max_splits, hipStream_t st,
+                       unsigned head_dim) {
+    if (!tiles || max_splits <= 1) return G4_OK;
+    return head_dim == 512 ? launch_token_merge_hd<512>(a, tiles, shift, max_splits, st)
+                           : launch_token_merge_hd<256>(a, tiles, shift, max_splits, st);
 }
 
 // attn.linearOut after a decode step (src/engine.ts:2096, the projection that

@@ -111,6 +111,12 @@ struct DecodeArgs {
 // head_dim: 256 or 512.
 int launch_decode_merge(const DecodeArgs& a, unsigned n_entries, unsigned max_splits, hipStream_t st,
                         unsigned head_dim = 256);
+// The same merge for prefill tokens: a.table lists `tiles` query tiles of up to
+// 2^shift tokens (pad: how many; out: the first one's attnOut, the next ones'
+// num_kv_heads * group * head_dim floats apart; n_splits records per token from
+// split_base on).
+int launch_token_merge(const DecodeArgs& a, unsigned tiles, unsigned shift, unsigned max_splits, hipStream_t st,
+                       unsigned head_dim);
 // The merges of a token's head_dim-512 step plan (a: more than 8 parts per
 // entry) and head_dim-256 plan (b: at most 8, group 4 or 8) in one launch, with
 // the bits of the two separate merges. Returns 1, launching nothing, when the

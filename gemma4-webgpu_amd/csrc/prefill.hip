@@ -1029,7 +1029,7 @@ struct PrefillPlanRep {
     char* ws;
     uint32_t n_entries;
     uint32_t n_work;
-    uint32_t n_merge;      // merge entries (tokens of split tiles)
+    uint32_t n_merge;      // merge entries (split tiles)
     uint32_t max_parts;
     uint16_t num_q_heads;
     uint16_t num_kv_heads;
@@ -1154,10 +1154,8 @@ int build(const g4_prefill_entry* ents, uint32_t n, uint32_t nqh, uint32_t nkh, 
                 items.push_back(Item{PrefillWorkDev{i, t, b0, b1, p, parts, base, 0}, b1 - b0});
             }
             if (parts > 1) {
-                for (uint32_t tk = 0; tk < ntok; tk++)
-                    merge->push_back(DecodeEntryDev{nullptr, nullptr, nullptr,
-                                                    e.out + (uint64_t)(tok0 + tk) * nqh * hd, 0, 0,
-                                                    base + tk * parts, parts, 0.0f, 0});
+                merge->push_back(DecodeEntryDev{nullptr, nullptr, nullptr, e.out + (uint64_t)tok0 * nqh * hd, 0, 0, base,
+                                                parts, 0.0f, ntok});
                 slots += (uint64_t)ntok * parts;
                 *max_parts = std::max(*max_parts, parts);
             }
@@ -1357,7 +1355,8 @@ static int prefill_run(const g4_decode_plan* plan, void* stream, hipEvent_t star
     m.group = a.group;
     m.part_ml = a.part_ml;
     m.part_o = a.part_o;
-    return launch_decode_merge(m, r.n_merge, r.max_parts, st, r.head_dim);
+    // tokens per tile: kPfRows / group, a power of two (the group divides 32)
+    return launch_token_merge(m, r.n_merge, (unsigned)__builtin_ctz(kPfRows / a.group), r.max_parts, st, r.head_dim);
 }
 
 int g4_attn_prefill_run(const g4_decode_plan* plan, void* stream) { return prefill_run(plan, stream, nullptr, nullptr); }
