@@ -152,7 +152,8 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
         // with. Absent tables are replaced by valid dummy addresses (the values
         // are not used).
         const float* rcs = ent.rope_cs;
-        const bool host_cs = rcs && adv == 0;  // uniform
+        const bool eval = ent.flags & kRopeEval;  // uniform: rcs is the inverse frequencies
+        const bool host_cs = rcs && adv == 0 && !eval;  // uniform
         const float* rsrc = host_cs ? rcs : ent.q;
         RopeLane<PJ> rl;
 #pragma unroll
@@ -165,7 +166,7 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
         const uint32_t fbits = ldg<uint16_t>((apply_divisor ? ent.rope_freqs : ent.q_weight) + pair);
         float inv_l[PJ];  // this lane's pairs' inverse frequencies from the set (advanced plans)
 #pragma unroll
-        for (int p = 0; p < PJ; p++) inv_l[p] = ldg<float>((rcs ? rcs + HD : ent.q) + lane + 64 * p);
+        for (int p = 0; p < PJ; p++) inv_l[p] = ldg<float>((rcs ? rcs + (eval ? 0 : HD) : ent.q) + lane + 64 * p);
         float xq[kQPerWave][J];
 #pragma unroll
         for (int r = 0; r < kQPerWave; r++) {
@@ -203,7 +204,7 @@ __device__ __forceinline__ void attn_step_body(const StepWorkDev* __restrict__ w
         __builtin_amdgcn_sched_barrier(0);  // keep every request above ahead of the arithmetic below
 
         // ---- q heads straight into the score operand; the current row's k and v ----
-        if (rcs && !host_cs) {  // uniform: each lane evaluates its own pairs at the advanced position,
+        if (rcs && !host_cs) {  // uniform: each lane evaluates its own pairs at the (advanced) position,
             // cos and sin of the f32 angle in f64 rounded to f32, as the host evaluates a prepared one
 #pragma unroll
             for (int p = 0; p < PJ; p++) f64_cos_sin((float)position * inv_l[p], rl.c[p], rl.s[p]);
@@ -363,6 +364,16 @@ namespace {
 
 constexpr uint32_t kStepMagic = 0x67345354u;
 
+// From this many RoPE factor sets on, most of them one entry's alone (the
+// sequences of a batch, each at its own position), a plan carries the inverse
+// frequencies and the kernel evaluates the factors, under its first tile's
+// latency. A layer stack's entries share one or two sets, which the host
+// evaluates and the kernel loads. Planned and run per token (us, host factors / so):
+// 8 sequences of 100 to 1000 rows 17.1 / 13.9, 16 to 3000 rows 23.2 / 17.5, 64 of 100
+// to 600 rows 56.7 / 16.7, 64 of 1K to 32K rows 188.3 / 184.9; 64 at head_dim 512 to
+// 3000 rows 101.4 / 57.9 (the evaluation on the host and 1 KB more to upload per set).
+constexpr uint32_t kStepRopeEvalSets = 4;
+
 struct StepPlanRep {
     char* tables;   // the plan's tables region (work items | merge table | entry table | RoPE factors)
     char* part_ml;  // its partial records: (m, l) pairs, then the o rows at step_part_o_offset()
@@ -447,8 +458,10 @@ int g4_attn_step_prepare(const g4_step_entry* entries, uint32_t n_entries, uint3
     const StepLayout L = step_layout(n_entries, num_kv_heads, G, head_dim);
     char* ws = static_cast<char*>(workspace);
     static thread_local StepPlanHost ph;  // the planner's storage, kept between the thread's prepares
+    StepTuning tune;
+    tune.rope_eval_sets = kStepRopeEvalSets;
     char err[256];
-    rc = plan_step(entries, n_entries, num_q_heads, num_kv_heads, head_dim, device_cus(), StepTuning{},
+    rc = plan_step(entries, n_entries, num_q_heads, num_kv_heads, head_dim, device_cus(), tune,
                    ws + L.tables, &ph, err, sizeof err);
     if (rc) return fail(rc, "%s", err);
     rc = stage_upload(ws + L.tables, ph.blob.data(), ph.blob.size(), as_stream(stream));  // the tables in one copy

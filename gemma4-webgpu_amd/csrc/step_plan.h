@@ -94,6 +94,9 @@ struct StepTuning {
     int waves = 0;       // 4 or 8 waves per workgroup (head_dim 256)
     int wgs_per_cu = 0;  // workgroups per CU
     int max_wgs = 0;     // cap on the workgroups of the launch
+    // Inverse frequencies in place of the RoPE factors (kRopeEval) when a plan has at least this many
+    // factor sets and fewer than two entries per set (0 = never)
+    uint32_t rope_eval_sets = 0;
 };
 
 struct StepPlanHost {
@@ -422,15 +425,27 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
     const size_t off_rope = off_ents + align256(n_entries * sizeof(DecodeEntryDev));
     // Each distinct pair's factors: a set placed by an earlier plan of the share, or one of this blob's.
     const float* rope_base = reinterpret_cast<const float*>(tables + off_rope);
+    const bool rope_eval = !share && tune.rope_eval_sets && ph.rope_keys.size() >= tune.rope_eval_sets &&
+                           2 * ph.rope_keys.size() > n_entries;
     size_t rope_sets = 0;
+    if (rope_eval) {  // one set per table, at no position: the pairs are looked up again without it
+        ph.rope_keys.clear();
+        ph.rope_slot.assign(ph.rope_slot.size(), 0u);
+        for (uint32_t i = 0; i < n_entries; i++)
+            if (ph.rope_idx[i] != ~0u) {
+                ph.rope_idx[i] = rope_pair_index(ph, entries[i].rope_inv_freq_host, 0);
+                ph.tab[i].flags |= kRopeEval;
+            }
+    }
+    const uint64_t rope_floats = rope_eval ? head_dim / 2 : rope_set_floats(head_dim);
     ph.rope_dev.resize(ph.rope_keys.size());
     ph.rope_set.resize(ph.rope_keys.size());
     for (size_t k = 0; k < ph.rope_keys.size(); k++) {
         const float* shared = share ? share->find(ph.rope_keys[k]) : nullptr;
         ph.rope_set[k] = shared ? ~0u : (uint32_t)rope_sets++;
-        ph.rope_dev[k] = shared ? shared : rope_base + (size_t)ph.rope_set[k] * rope_set_floats(head_dim);
+        ph.rope_dev[k] = shared ? shared : rope_base + (size_t)ph.rope_set[k] * rope_floats;
     }
-    ph.blob.resize(off_rope + rope_sets * rope_set_floats(head_dim) * sizeof(float));
+    ph.blob.resize(off_rope + rope_sets * rope_floats * sizeof(float));
     char* blob = ph.blob.data();
     memset(blob + n_work * sizeof(StepWorkDev), 0, off_merge - n_work * sizeof(StepWorkDev));
     memset(blob + off_merge + n_merge * sizeof(DecodeEntryDev), 0, off_ents - off_merge - n_merge * sizeof(DecodeEntryDev));
@@ -442,7 +457,11 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
         float* rope = reinterpret_cast<float*>(blob + off_rope);
         for (size_t k = 0; k < ph.rope_keys.size(); k++) {
             if (ph.rope_set[k] == ~0u) continue;  // placed by an earlier plan
-            float* set = rope + (size_t)ph.rope_set[k] * rope_set_floats(head_dim);
+            float* set = rope + (size_t)ph.rope_set[k] * rope_floats;
+            if (rope_eval) {
+                memcpy(set, ph.rope_keys[k].first, head_dim / 2 * sizeof(float));
+                continue;
+            }
             rope_factors(ph.rope_keys[k].first, ph.rope_keys[k].second, head_dim / 2, set);
             memcpy(set + head_dim, ph.rope_keys[k].first, head_dim / 2 * sizeof(float));  // the inverse frequencies
             if (share) share->add(ph.rope_keys[k], ph.rope_dev[k]);

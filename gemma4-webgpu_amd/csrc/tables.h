@@ -34,14 +34,15 @@ struct StepEntryDev {
     const uint16_t* k_weight;
     const uint16_t* rope_freqs;
     const float* rope_cs;  // RoPE set of this token: [cos x HD/2][sin x HD/2] at `position` (host-computed),
-                           // then the inverse frequencies [HD/2] (for later positions); or nullptr
+                           // then the inverse frequencies [HD/2] (for later positions; those alone
+                           // with kRopeEval); or nullptr
     uint16_t* k_cache;  // [rows][num_kv_heads][HD]
     uint16_t* v_cache;
     float* out;         // attnOut [num_kv_heads][group][HD]
     uint32_t key_end;   // one past the last attended row; the current row is key_end - 1
     uint32_t n_parts;   // workgroups on this entry
     uint32_t position;  // RoPE position
-    uint32_t flags;     // kStoreKv | kRowCached | kApplyDivisor | kQReady
+    uint32_t flags;     // kStoreKv | kRowCached | kApplyDivisor | kRopeEval | kQReady | kQReady
     float theta;
     uint32_t window;    // sliding window (0 = full): rows [key_end - window, key_end) when key_end > window
     float qscale;       // attention scale * log2(e)
@@ -51,6 +52,7 @@ struct StepEntryDev {
 constexpr uint32_t kStoreKv = 1;       // write the current row's k and v to the caches
 constexpr uint32_t kRowCached = 2;     // the current row is already in the cache: read it like the others
 constexpr uint32_t kApplyDivisor = 4;  // RoPE frequencies divided by rope_freqs (global layers)
+constexpr uint32_t kRopeEval = 16;     // rope_cs holds the inverse frequencies alone: the kernel evaluates the factors
 constexpr uint32_t kQReady = 8;        // q holds the post-norm, post-RoPE query: read as is
 
 // First attended row of an entry whose rows end at key_end. (constexpr: the
