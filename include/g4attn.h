@@ -415,9 +415,9 @@ int g4_attn_step_run_attention_timed(const g4_decode_plan* plan, void* stream, v
  * ones' tail). The plans (either order) come from separate prepares with
  * separate workspaces. Each plan's merge then runs as usual
  * (g4_attn_step_run_merge); g4_attn_step_run_pair does all three. The
- * head_dim-256 entries are computed by 4-wave workgroups whatever the plan's
+ * head_dim-256 entries are computed by 8-wave workgroups whatever the plan's
  * own form, so their results agree with g4_attn_step_run's to rounding, not
- * bit for bit, when that plan took 8-wave workgroups. No counterpart in the
+ * bit for bit, when that plan took 4-wave workgroups. No counterpart in the
  * reference (one dispatch per kernel per layer, src/engine.ts:2056-2095). */
 int g4_attn_step_run_attention_pair(const g4_decode_plan* plan_1, const g4_decode_plan* plan_2, void* stream);
 int g4_attn_step_run_attention_pair_timed(const g4_decode_plan* plan_1, const g4_decode_plan* plan_2, void* stream,
