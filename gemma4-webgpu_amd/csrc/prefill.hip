@@ -1119,19 +1119,30 @@ int build(const g4_prefill_entry* ents, uint32_t n, uint32_t nqh, uint32_t nkh, 
         // Parts about 1.15x the keys per CU of the whole call (one workgroup per CU): long query
         // tiles split so that the longest item stays near a CU's share, short ones stay whole
         // (every extra part costs a record write and its merge). prefill4k: 3008 keys; measured
-        // 168 us against 177 us at 1536 and 183 us at 3840.
-        uint64_t w = 0;
+        // 168 us against 177 us at 1536 and 183 us at 3840. At least 256 keys, or 160 where parts of
+        // 256 would leave two thirds of the CUs idle and a merge is due anyway (a longer tile than
+        // 256): an item's time is its fixed cost and ~1 us per 32 keys. Measured, 256 / 160 (us, kept
+        // plans): 30 tokens after 2000 cached 26.7 / 25.1, 80 after 800 27.0 / 25.6, 5 after 3000 on one
+        // layer 23.8 / 21.6; head_dim 512: 8 after 1500 35.4 / 30.2, 80 after 500 35.5 / 32.5. With more
+        // items the longer merges cost more: head_dim 512, 500 tokens 34.9 / 35.8; 143 tokens alone
+        // (no merge at 256) 20.2, 22.9 in parts of 128.
+        uint64_t w = 0, items256 = 0;
+        uint32_t longest = 0;
         for (uint32_t i = 0; i < n; i++) {
             const g4_prefill_entry& e = ents[i];
             const uint32_t tiles = (uint32_t)(((uint64_t)e.n_tokens * G + kPfRows - 1) / kPfRows);
             for (uint32_t t = 0; t < tiles; t++) {
                 uint32_t kb, ke;
                 tile_keys(e, G, t, &kb, &ke);
-                w += ke - (kb & ~(uint32_t)(kPfKeys - 1));
+                const uint32_t nk = ke - (kb & ~(uint32_t)(kPfKeys - 1));
+                w += nk;
+                items256 += (nk + 255) / 256;
+                longest = std::max(longest, nk);
             }
         }
         const uint64_t share = w * nkh * (hd / 256) * 115 / (100 * (uint64_t)device_cus());  // head_dim 512: two halves
-        part_keys = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(share, 256), 1u << 30);
+        const uint64_t least = longest > 256 && 3 * items256 * nkh * (hd / 256) <= device_cus() ? 160 : 256;
+        part_keys = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(share, least), 1u << 30);
         part_keys = (part_keys + kPfKeys - 1) / kPfKeys * kPfKeys;
     }
     for (uint32_t i = 0; i < n; i++) {
