@@ -1074,8 +1074,12 @@ struct VtPlan {
     uint32_t total_blocks = 0;
 };
 
-// Work list, merge list and workspace layout for a set of entries.
-int build(const g4_prefill_entry* ents, uint32_t n, uint32_t nqh, uint32_t nkh, uint32_t hd,
+// The fewest keys of a part, where the call's work does not ask for more (build has the rule).
+constexpr uint32_t kPfPartKeys = 256, kPfShortPartKeys = 160;
+
+// Work list, merge list and workspace layout for a set of entries. short_parts: parts of
+// kPfShortPartKeys are allowed.
+int build(const g4_prefill_entry* ents, uint32_t n, uint32_t nqh, uint32_t nkh, uint32_t hd, bool short_parts,
           std::vector<PrefillEntryDev>* tab, std::vector<PrefillWorkDev>* work, std::vector<uint32_t>* lists,
           std::vector<DecodeEntryDev>* merge, uint32_t* max_parts, Layout* L, VtPlan* vp) {
     const uint32_t G = nqh / nkh;
@@ -1126,7 +1130,7 @@ int build(const g4_prefill_entry* ents, uint32_t n, uint32_t nqh, uint32_t nkh, 
         // layer 23.8 / 21.6; head_dim 512: 8 after 1500 35.4 / 30.2, 80 after 500 35.5 / 32.5. With more
         // items the longer merges cost more: head_dim 512, 500 tokens 34.9 / 35.8; 143 tokens alone
         // (no merge at 256) 20.2, 22.9 in parts of 128.
-        uint64_t w = 0, items256 = 0;
+        uint64_t w = 0, long_items = 0;  // long_items: with parts of kPfPartKeys
         uint32_t longest = 0;
         for (uint32_t i = 0; i < n; i++) {
             const g4_prefill_entry& e = ents[i];
@@ -1136,12 +1140,13 @@ int build(const g4_prefill_entry* ents, uint32_t n, uint32_t nqh, uint32_t nkh, 
                 tile_keys(e, G, t, &kb, &ke);
                 const uint32_t nk = ke - (kb & ~(uint32_t)(kPfKeys - 1));
                 w += nk;
-                items256 += (nk + 255) / 256;
+                long_items += (nk + kPfPartKeys - 1) / kPfPartKeys;
                 longest = std::max(longest, nk);
             }
         }
         const uint64_t share = w * nkh * (hd / 256) * 115 / (100 * (uint64_t)device_cus());  // head_dim 512: two halves
-        const uint64_t least = longest > 256 && 3 * items256 * nkh * (hd / 256) <= device_cus() ? 160 : 256;
+        const bool few = longest > kPfPartKeys && 3 * long_items * nkh * (hd / 256) <= device_cus();
+        const uint64_t least = short_parts && few ? kPfShortPartKeys : kPfPartKeys;
         part_keys = (uint32_t)std::min<uint64_t>(std::max<uint64_t>(share, least), 1u << 30);
         part_keys = (part_keys + kPfKeys - 1) / kPfKeys * kPfKeys;
     }
@@ -1254,7 +1259,7 @@ int g4_attn_prefill_workspace_size(const g4_prefill_entry* entries, uint32_t n_e
     uint32_t mp;
     Layout L;
     VtPlan vp;
-    rc = build(entries, n_entries, num_q_heads, num_kv_heads, head_dim, &tab, &work, &lists, &merge, &mp, &L, &vp);
+    rc = build(entries, n_entries, num_q_heads, num_kv_heads, head_dim, true, &tab, &work, &lists, &merge, &mp, &L, &vp);
     if (rc) return rc;
     *bytes = L.total;
     return G4_OK;
@@ -1273,8 +1278,15 @@ int g4_attn_prefill_prepare(const g4_prefill_entry* entries, uint32_t n_entries,
     uint32_t max_parts;
     Layout L;
     VtPlan vp;
-    rc = build(entries, n_entries, num_q_heads, num_kv_heads, head_dim, &tab, &work, &lists, &merge, &max_parts, &L, &vp);
-    if (rc) return rc;
+    // Short parts take more records: a workspace sized for a longer prompt, which keeps the longer parts, can hold
+    // fewer of them than a short prompt would use. The short prompt then takes the longer parts too.
+    for (bool short_parts : {true, false}) {
+        merge.clear();
+        rc = build(entries, n_entries, num_q_heads, num_kv_heads, head_dim, short_parts, &tab, &work, &lists, &merge,
+                   &max_parts, &L, &vp);
+        if (rc) return rc;
+        if (workspace_bytes >= L.total) break;
+    }
     if (max_parts > 8192) return fail(G4_EINVAL, "attnPrefill: %u key parts per tile (max 8192)", max_parts);
     if (!workspace || workspace_bytes < L.total)
         return fail(G4_ENOSPC, "attnPrefill: workspace %zu bytes < %zu needed", workspace_bytes, L.total);

@@ -480,6 +480,11 @@ typedef struct g4_prefill_entry {
     uint32_t vt_rows;         /* rows the V^T cache was sized for (the prompt prep's max_seq_len) */
 } g4_prefill_entry;
 
+/* Bytes for these entries with the key parts that are the fastest for them. More query tiles over the same keys
+ * can take longer parts and so fewer bytes. A prepare whose workspace is too small for short parts (160 keys, of
+ * prompts that leave most of the GPU idle) falls back to parts of at least 256 keys, and the attention rounds in
+ * that partition's order; it returns G4_ENOSPC only when those do not fit either. A workspace for prompts of
+ * several lengths is sized for the largest of their sizes. */
 int g4_attn_prefill_workspace_size(const g4_prefill_entry* entries, uint32_t n_entries, uint32_t num_q_heads,
                                    uint32_t num_kv_heads, uint32_t head_dim, size_t* bytes);
 int g4_attn_prefill_prepare(const g4_prefill_entry* entries, uint32_t n_entries, uint32_t num_q_heads,
