@@ -47,6 +47,7 @@
 #include <vector>
 
 #include "decode_core.h"
+#include "launch_rules.h"
 
 namespace g4 {
 
@@ -1030,7 +1031,8 @@ struct PrefillPlanRep {
     uint32_t n_entries;
     uint32_t n_work;
     uint32_t n_merge;      // merge entries (split tiles)
-    uint32_t max_parts;
+    uint16_t max_parts;    // at most kPfMaxParts
+    uint16_t merge_shift;  // token_merge_shift of the split tiles
     uint16_t num_q_heads;
     uint16_t num_kv_heads;
     uint16_t head_dim;     // 256 or 512
@@ -1076,6 +1078,7 @@ struct VtPlan {
 
 // The fewest keys of a part, where the call's work does not ask for more (build has the rule).
 constexpr uint32_t kPfPartKeys = 256, kPfShortPartKeys = 160;
+constexpr uint32_t kPfMaxParts = 8192;  // of a query tile
 
 // Work list, merge list and workspace layout for a set of entries. short_parts: parts of
 // kPfShortPartKeys are allowed.
@@ -1287,7 +1290,8 @@ int g4_attn_prefill_prepare(const g4_prefill_entry* entries, uint32_t n_entries,
         if (rc) return rc;
         if (workspace_bytes >= L.total) break;
     }
-    if (max_parts > 8192) return fail(G4_EINVAL, "attnPrefill: %u key parts per tile (max 8192)", max_parts);
+    if (max_parts > kPfMaxParts)
+        return fail(G4_EINVAL, "attnPrefill: %u key parts per tile (max %u)", max_parts, kPfMaxParts);
     if (!workspace || workspace_bytes < L.total)
         return fail(G4_ENOSPC, "attnPrefill: workspace %zu bytes < %zu needed", workspace_bytes, L.total);
     if (L.vt >= (1ull << 32)) return fail(G4_EINVAL, "attnPrefill: workspace layout exceeds 4 GiB");
@@ -1312,7 +1316,10 @@ int g4_attn_prefill_prepare(const g4_prefill_entry* entries, uint32_t n_entries,
     r.n_entries = n_entries;
     r.n_work = (uint32_t)work.size();
     r.n_merge = (uint32_t)merge.size();
-    r.max_parts = max_parts;
+    r.max_parts = (uint16_t)max_parts;
+    uint32_t tile_tokens = 0;
+    for (const DecodeEntryDev& m : merge) tile_tokens = std::max(tile_tokens, m.pad);
+    r.merge_shift = (uint16_t)token_merge_shift(tile_tokens);
     r.num_q_heads = (uint16_t)num_q_heads;  // at most 8 per kv head (checked); kv heads below 2^16
     r.num_kv_heads = (uint16_t)num_kv_heads;
     r.head_dim = (uint16_t)head_dim;
@@ -1378,8 +1385,7 @@ static int prefill_run(const g4_decode_plan* plan, void* stream, hipEvent_t star
     m.group = a.group;
     m.part_ml = a.part_ml;
     m.part_o = a.part_o;
-    // tokens per tile: kPfRows / group, a power of two (the group divides 32)
-    return launch_token_merge(m, r.n_merge, (unsigned)__builtin_ctz(kPfRows / a.group), r.max_parts, st, r.head_dim);
+    return launch_token_merge(m, r.n_merge, r.merge_shift, r.max_parts, st, r.head_dim);
 }
 
 int g4_attn_prefill_run(const g4_decode_plan* plan, void* stream) { return prefill_run(plan, stream, nullptr, nullptr); }

@@ -1,0 +1,20 @@
+// Evaluates the launch rules (gemma4-webgpu_amd/csrc/launch_rules.h) for tests/test_launch_rules.py: reads
+// "<rule> <arguments>" lines and prints one value a line.
+#include <stdio.h>
+
+#include <iostream>
+#include <string>
+
+#include "../gemma4-webgpu_amd/csrc/launch_rules.h"
+
+int main() {
+    std::string rule;
+    while (std::cin >> rule) {
+        uint32_t a = 0;
+        if (rule == "token_merge_shift" && std::cin >> a)
+            printf("%u\n", g4::token_merge_shift(a));
+        else
+            return fprintf(stderr, "unknown rule %s\n", rule.c_str()), 1;
+    }
+    return 0;
+}
