@@ -77,8 +77,8 @@ struct StepSmem {
 // 128 of a wave's 256 registers. At 512 one 4-wave workgroup per CU with 32-row
 // tiles at one wave per SIMD has nothing to run while its tile's loads are out,
 // and two query heads per wave in the prologue (us per step of one layer, that
-// form / this: 1023 rows 12.9 / 10.8, 4096 13.2 / 12.5, 32768 24.6 / 24.2, 100000
-// 45.8 / 44.1; a token of both head_dims with shared caches at 32768 70.4 / 64.2).
+// form / this: 1023 rows 13.0 / 10.5, 4096 13.4 / 12.4, 32768 24.7 / 23.3, 100000
+// 46.0 / 43.4; a token of both head_dims with shared caches at 32768 70.4 / 63.0).
 //
 // The arguments are scalars and pointers (not one struct) so that they are
 // preloaded into SGPRs at wave start (the file is compiled with kernarg
