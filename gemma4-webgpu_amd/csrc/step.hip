@@ -342,7 +342,7 @@ union StepPairSmem {
     StepSmem<8, 256> b;
 };
 
-template <bool KEEP>
+template <bool KEEP_A, bool KEEP_B>
 __global__ __launch_bounds__(512, 1) void k_attn_step_pair(
     const StepWorkDev* __restrict__ work_a, float* ml_a, float* o_a, uint32_t nkh_a, uint32_t group_a, uint32_t adv_a,
     uint32_t wgs_a, const StepWorkDev* __restrict__ work_b, float* ml_b, float* o_b, uint32_t nkh_b, uint32_t group_b,
@@ -350,9 +350,9 @@ __global__ __launch_bounds__(512, 1) void k_attn_step_pair(
     __shared__ StepPairSmem sm;
     const unsigned x = blockIdx.x, y = blockIdx.y;
     if (x < wgs_a) {  // uniform
-        if (y < nkh_a) attn_step_body<8, 512, KEEP>(work_a, ml_a, o_a, nkh_a, group_a, adv_a, x, y, sm.a);
+        if (y < nkh_a) attn_step_body<8, 512, KEEP_A>(work_a, ml_a, o_a, nkh_a, group_a, adv_a, x, y, sm.a);
     } else if (y < nkh_b) {
-        attn_step_body<8, 256, KEEP>(work_b, ml_b, o_b, nkh_b, group_b, adv_b, x - wgs_a, y, sm.b);
+        attn_step_body<8, 256, KEEP_B>(work_b, ml_b, o_b, nkh_b, group_b, adv_b, x - wgs_a, y, sm.b);
     }
 }
 
@@ -599,7 +599,10 @@ static int launch_attention_pair(const g4_decode_plan* plan_1, const g4_decode_p
             G4_LAUNCH(kernel, grid, dim3(512), 0, st, wa, ml(a), po(a), (uint32_t)a.num_kv_heads, (uint32_t)a.group,
                       a.adv, (uint32_t)a.n_wgs, wb, ml(b), po(b), (uint32_t)b.num_kv_heads, (uint32_t)b.group, b.adv);
     };
-    a.keep_rows || b.keep_rows ? launch(k_attn_step_pair<true>) : launch(k_attn_step_pair<false>);
+    if (a.keep_rows)
+        b.keep_rows ? launch(k_attn_step_pair<true, true>) : launch(k_attn_step_pair<true, false>);
+    else
+        b.keep_rows ? launch(k_attn_step_pair<false, true>) : launch(k_attn_step_pair<false, false>);
     G4_CHECK_LAUNCH("attnStepPair");
     return G4_OK;
 }

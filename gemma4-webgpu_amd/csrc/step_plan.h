@@ -30,6 +30,7 @@ namespace g4 {
 constexpr unsigned kStepMaxWgs = 1024;
 constexpr unsigned kXcds = 8;            // workgroups go round the XCDs in index order
 constexpr unsigned kStepOneWgTiles = 16;  // one workgroup per CU up to this many tiles each
+constexpr unsigned kStepKeepShare = 8;    // rows are kept from 1/8 of the tiles on (StepPlanHost::keep_rows)
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -104,12 +105,19 @@ struct StepPlanHost {
     uint32_t n_wgs = 0;      // workgroups (work items)
     uint32_t n_merge = 0;    // entries in the merge table
     uint32_t max_parts = 0;  // largest part count of an entry
-    // The attention kernel reads rows with ordinary loads: where entries share rows
-    // (a row is read again, from L2 or the MALL). Otherwise a row is read once per
-    // token and streamed: a step larger than the MALL is faster so (64 sequences of
-    // 1K to 32K rows 188 us streamed, 204 kept), and a smaller one does not write back
-    // what earlier work left dirty there (35 layers at 8192, caches full of written
-    // lines: 23.6 us streamed, 34.9 kept; full of read ones: 23.2 and 22.5).
+    // The attention kernel reads rows with ordinary loads, which L2 and the MALL keep:
+    // where at least an eighth of the step's tiles are rows that an earlier entry of the
+    // step reads too (kStepKeepShare). Otherwise rows are streamed: a step larger than the
+    // MALL is faster so, and a smaller one does not write back what earlier work left dirty
+    // there (35 layers at 8192, caches full of written lines: 23.6 us streamed, 34.9 kept;
+    // full of read ones: 23.2 and 22.5). Measured with some entries reading others' rows,
+    // caches full of read lines, kept / streamed (us; the share in brackets): 64 sequences
+    // of 1K to 32K rows 192.4 / 176.5 [0.01], 174.8 / 175.2 [0.11], 166.5 / 168.9 [0.15],
+    // 118.5 / 157.4 [0.5]; 35 of 8192 rows 57.6 / 55.2 [0.03], 53.4 / 53.1 [0.11],
+    // 51.9 / 52.5 [0.14], 41.1 / 47.9 [0.49]; head_dim 512, 32 of 1K to 20K rows
+    // 129.1 / 125.6 [0.02], 119.1 / 123.8 [0.14]. After written lines kept rows lose up to
+    // a share of two thirds (35 of 8192 rows, 0.49: 65.4 / 47.0); what a decode loop leaves
+    // there is read ones, its weights.
     bool keep_rows = false;
     uint32_t parts = 0;      // partial-record slots in use
     size_t off_merge = 0;    // byte offsets in the tables blob
@@ -260,16 +268,17 @@ inline uint32_t rope_pair_index(StepPlanHost& ph, const float* table, uint32_t p
 
 // Groups the entries that read the same cache rows (KV-sharing layers of one
 // token): kv_first[i] is the first entry with entry i's caches and row range,
-// kv_next[i] the next one of its group (~0: the last). Returns whether any
-// group has two entries. Open addressing as in rope_pair_index.
-inline bool kv_groups(StepPlanHost& ph) {
+// kv_next[i] the next one of its group (~0: the last). Returns the tiles of the
+// entries that are not the first of their group (0: no group has two entries).
+// Open addressing as in rope_pair_index.
+inline uint64_t kv_groups(StepPlanHost& ph) {
     const uint32_t n = (uint32_t)ph.tab.size();
     size_t slots = 16;
     while (slots < 2 * (size_t)n) slots *= 2;
     ph.kv_slot.assign(slots, 0u);
     ph.kv_first.resize(n);
     ph.kv_next.assign(n, ~0u);
-    bool shared = false;
+    uint64_t again = 0;
     for (uint32_t i = 0; i < n; i++) {
         const StepEntryDev& e = ph.tab[i];
         const uint64_t h = (reinterpret_cast<uintptr_t>(e.k_cache) >> 4) * 0x9E3779B97F4A7C15ull ^
@@ -282,7 +291,7 @@ inline bool kv_groups(StepPlanHost& ph) {
                     continue;
                 ph.kv_first[i] = ph.kv_first[v - 1];
                 ph.kv_next[v - 1] = i;
-                shared = true;
+                again += ph.tiles[i];
             } else {
                 ph.kv_first[i] = i;
             }
@@ -290,7 +299,7 @@ inline bool kv_groups(StepPlanHost& ph) {
             break;
         }
     }
-    return shared;
+    return again;
 }
 
 // Checks the step's arguments and plans it. `tables` is the device address of
@@ -472,7 +481,8 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
     DecodeEntryDev* merge = reinterpret_cast<DecodeEntryDev*>(blob + off_merge);
     DecodeEntryDev* ents = reinterpret_cast<DecodeEntryDev*>(blob + off_ents);
     uint32_t part_next = 0;
-    const bool shared = kv_groups(ph);
+    const uint64_t again = kv_groups(ph);  // tiles whose rows another entry reads too
+    const bool shared = again != 0;
     ph.part_base.resize(n_entries);
     for (uint32_t i = 0; i < n_entries; i++) {
         StepEntryDev& d = ph.tab[i];
@@ -542,7 +552,7 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
                 }
             }
         }
-    ph.keep_rows = shared;
+    ph.keep_rows = again * kStepKeepShare >= T;
     ph.waves = waves;
     ph.n_wgs = (uint32_t)n_work;
     ph.n_merge = n_merge;

@@ -2,7 +2,8 @@
 // (gemma4-webgpu_amd/csrc/step_plan.h), built with g++ by tests/test_kv_share_plan.py. Random steps whose
 // entries read a few caches over a few row ranges: every part of every entry is planned exactly once with the
 // rows of the plan without sharing, and the items of one part of a group sit on one XCD (workgroup index mod 8)
-// unless the group straddles the end of an XCD's workgroups. Prints "ok <steps> <shared steps>".
+// unless the group straddles the end of an XCD's workgroups. Rows are read with ordinary loads where enough of the
+// step's tiles are read again. Prints "ok <steps> <shared steps> <steps that keep rows>".
 #include <stdio.h>
 
 #include <map>
@@ -20,7 +21,7 @@ int main() {
     static char dev[1 << 16];
     uint16_t* base = reinterpret_cast<uint16_t*>(dev);
     float* f = reinterpret_cast<float*>(dev);
-    int shared_steps = 0, steps = 3000;
+    int shared_steps = 0, kept_steps = 0, steps = 3000;
     for (int it = 0; it < steps; it++) {
         const uint32_t n = pick(1, 40), hd = pick(0, 1) ? 512 : 256, caches = pick(1, 6);
         std::vector<g4_step_entry> e(n);
@@ -62,7 +63,17 @@ int main() {
         if (a != b || a.size() != ph.n_wgs) return printf("FAIL items %d\n", it), 1;
         bool shared = false;
         for (auto& g : groups) shared |= g.second.size() > 1;
-        if (ph.keep_rows != shared) return printf("FAIL keep_rows %d\n", it), 1;
+        // Rows are kept where an eighth of the tiles or more read rows that an earlier entry reads.
+        uint64_t total = 0, again = 0;
+        std::set<std::tuple<const void*, const void*, uint32_t, uint32_t>> seen;
+        for (const auto& s : e) {
+            const uint32_t first = s.sliding_window && s.seq_len > s.sliding_window ? s.seq_len - s.sliding_window : 0;
+            const uint32_t tiles = (s.seq_len - first + 31) / 32;
+            total += tiles;
+            if (!seen.insert({s.k_cache, s.v_cache, s.seq_len, s.sliding_window}).second) again += tiles;
+        }
+        if (ph.keep_rows != (8 * again >= total)) return printf("FAIL keep_rows %d\n", it), 1;
+        kept_steps += ph.keep_rows;
         shared_steps += shared;
         size_t crossings = 0;
         for (auto& g : xcds) crossings += g.second.size() - 1;
@@ -71,6 +82,23 @@ int main() {
             for (uint32_t i = 0; i + 1 < ph.n_wgs; i++)
                 if (w[i].entry > w[i + 1].entry) return printf("FAIL order %d\n", it), 1;
     }
-    printf("ok %d %d\n", steps, shared_steps);
+    // One sequence twice in a large batch, and one short window shared beside long rows: streamed.
+    for (int window : {0, 1}) {
+        std::vector<g4_step_entry> e(64);
+        for (uint32_t i = 0; i < e.size(); i++) {
+            e[i].q = e[i].k = e[i].v = f;
+            e[i].q_weight = e[i].k_weight = base;
+            e[i].k_cache = e[i].v_cache = base + 8 * (i < 63 ? i : 5);
+            e[i].out = f;
+            e[i].seq_len = i < 63 ? 1000 + 200 * i : 2000;
+            e[i].sliding_window = window && (i == 5 || i == 63) ? 64 : 0;
+            e[i].scale = 1.0f;
+        }
+        StepPlanHost ph;
+        char err[256];
+        if (plan_step(e.data(), 64, 8, 1, 256, 256, StepTuning{}, dev, &ph, err, sizeof err)) return printf("FAIL %s\n", err), 1;
+        if (ph.kv_next[5] != 63 || ph.keep_rows) return printf("FAIL a small shared pair\n"), 1;
+    }
+    printf("ok %d %d %d\n", steps, shared_steps, kept_steps);
     return 0;
 }

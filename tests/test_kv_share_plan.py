@@ -15,5 +15,6 @@ def test_kv_share_order(tmp_path):
                     str(ROOT / "tests" / "kv_share_check.cpp"), "-o", str(exe)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stdout + out.stderr
-    _, steps, shared = out.stdout.split()
+    _, steps, shared, kept = out.stdout.split()
     assert int(shared) > int(steps) // 2
+    assert int(steps) // 4 < int(kept) < int(shared) - int(steps) // 40  # both sides of the rule
