@@ -17,4 +17,21 @@ inline unsigned token_merge_shift(uint32_t tile_tokens) {
     return s;
 }
 
+// Scores per thread of softmax's register form (4 or 16), or 0 for the loop
+// form. The register form's 1024 threads a head pay for their launch and their
+// exchange through LDS from 513 scores on (us in a replayed graph, loop / register:
+// 8 heads of 64 scores 3.2 / 3.9, of 400 4.5 / 4.6, of 513 5.0 / 4.7, of 2048
+// 7.3 / 4.9), and two such workgroups fill a CU where the loop form's 256 threads
+// run eight deep: above 256 heads the line is at 11/4 scores for each head of the launch
+// (512 heads of 1024 5.8 / 6.8, of 1500 7.9 / 7.2; 1024 heads of 2048 9.6 / 11.7, of 3000
+// 13.3 / 12.8), at 6 with 16 scores a thread, where one workgroup fills a CU (1024
+// heads of 5000 23.2 / 26.1, of 7000 32.4 / 26.7; 2048 heads of 7000 48.2 / 47.7).
+// Past 16384 scores LDS and the registers hold no more.
+inline unsigned softmax_scores_per_thread(uint32_t heads, uint32_t seq_len) {
+    if (seq_len <= 512 || seq_len > 16384) return 0;
+    const bool few = heads <= 256;
+    if (seq_len <= 4096) return few || 4ull * seq_len >= 11ull * heads ? 4 : 0;
+    return few || seq_len >= 6ull * heads ? 16 : 0;
+}
+
 }  // namespace g4

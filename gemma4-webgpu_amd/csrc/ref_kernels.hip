@@ -20,6 +20,7 @@
 // IEEE correctly rounded, and pow/sin/cos/exp return the f32 nearest to the
 // exact value (evaluated in f64), so results are reproducible bit for bit on
 // any IEEE machine that evaluates the same expressions.
+#include "launch_rules.h"
 #include "ref_math.h"
 
 namespace g4 {
@@ -504,17 +505,13 @@ int g4_softmax(float* scores, g4_softmax_params p, void* stream) {
     if (!scores) return fail(G4_EINVAL, "softmax: NULL scores");
     if (p.seq_len == 0) return fail(G4_EINVAL, "softmax: seq_len 0");
     if (p.num_heads == 0) return G4_OK;
-    if (p.seq_len <= 4 * kSoftThreads) {
+    const unsigned per_thread = softmax_scores_per_thread(p.num_heads, p.seq_len);
+    if (per_thread == 4)
         G4_LAUNCH(k_softmax_reg<4>, dim3(p.num_heads), dim3(kSoftThreads), 0, as_stream(stream), scores, p);
-        G4_CHECK_LAUNCH("softmax");
-        return G4_OK;
-    }
-    if (p.seq_len <= 16 * kSoftThreads) {  // up to the scores that LDS and the registers hold
+    else if (per_thread == 16)
         G4_LAUNCH(k_softmax_reg<16>, dim3(p.num_heads), dim3(kSoftThreads), 0, as_stream(stream), scores, p);
-        G4_CHECK_LAUNCH("softmax");
-        return G4_OK;
-    }
-    G4_LAUNCH(k_softmax, dim3(p.num_heads), dim3(kWG), 0, as_stream(stream), scores, p);
+    else
+        G4_LAUNCH(k_softmax, dim3(p.num_heads), dim3(kWG), 0, as_stream(stream), scores, p);
     G4_CHECK_LAUNCH("softmax");
     return G4_OK;
 }

@@ -28,3 +28,23 @@ def test_token_merge_columns(rule, tokens):
     """The columns cover the largest tile's tokens, and fewer than twice as many are launched."""
     columns = 1 << rule("token_merge_shift", tokens)
     assert tokens <= columns < 2 * tokens
+
+
+@pytest.mark.parametrize("heads,seq,form", [
+    # the loop form, measured the faster one
+    (8, 1, 0), (8, 64, 0), (8, 256, 0), (64, 512, 0), (512, 64, 0), (512, 300, 0), (512, 1024, 0), (1024, 100, 0),
+    (1024, 2048, 0), (2048, 100, 0), (2048, 2048, 0), (2048, 4096, 0), (1024, 5000, 0), (2048, 5000, 0), (8, 16385, 0),
+    # the register form, measured the faster one
+    (1, 513, 4), (8, 600, 4), (8, 1000, 4), (8, 4096, 4), (256, 1024, 4), (512, 1500, 4), (512, 2048, 4), (1024, 3000, 4), (1024, 4096, 4), (8, 4097, 16),
+    (8, 16384, 16), (512, 8192, 16), (1024, 7000, 16)])
+def test_softmax_form(rule, heads, seq, form):
+    assert rule("softmax_scores_per_thread", heads, seq) == form
+    if form:  # the register form holds the scores
+        assert seq <= 1024 * form
+
+
+def test_softmax_form_at_the_limits(rule):
+    for heads in (1, 256, 257, 2**31, 2**32 - 1):
+        for seq in (1, 512, 513, 4096, 4097, 16384, 16385, 2**32 - 1):
+            form = rule("softmax_scores_per_thread", heads, seq)
+            assert form in (0, 4, 16) and (not form or 512 < seq <= 1024 * form)
