@@ -456,21 +456,25 @@ __device__ __forceinline__ void wave_publish(DecodeSmem<HD, W>& sm, int wave, in
             o[i * 128 + 32] = n < 8 ? x[1] : x[3];
             __builtin_amdgcn_sched_barrier(0);
         }
-    } else {
+        if (n < 8 && g == 0) {
+            sm.m[wave][n] = m_run;
+            sm.l[wave][n] = l;
+        }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < NO; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = dpp_ror8_add(acc[i][j]);
+    if (n < 8) {
 #pragma unroll
         for (int i = 0; i < NO; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) acc[i][j] = dpp_ror8_add(acc[i][j]);
-        if (n < 8) {
-#pragma unroll
-            for (int i = 0; i < NO; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) sm.o[wave][i * 4 + j][g * 8 + n] = acc[i][j];
+            for (int j = 0; j < 4; j++) sm.o[wave][i * 4 + j][g * 8 + n] = acc[i][j];
+        if (g == 0) {
+            sm.m[wave][n] = m_run;
+            sm.l[wave][n] = l;
         }
-    }
-    if (n < 8 && g == 0) {
-        sm.m[wave][n] = m_run;
-        sm.l[wave][n] = l;
     }
 }
 
