@@ -34,4 +34,20 @@ inline unsigned softmax_scores_per_thread(uint32_t heads, uint32_t seq_len) {
     return few || seq_len >= 6ull * heads ? 16 : 0;
 }
 
+// attnOutput: whether its chain form takes `workgroups` (64 columns of a head
+// each) over seq_len rows on `cus` compute units. The form's products fill 129 KB of LDS,
+// so one workgroup runs per CU, and a round of them takes ~1.6 us + 4.4 ns a
+// row; the general form's dependent loads take ~107 ns a row whatever the
+// number of workgroups. Both meet near 16, 33, 74, 187 and 640 rows at 1, 2, 4, 8
+// and 16 rounds, and by 1024 rows at 32 (V then leaves the L2, and the general form
+// doubles). Measured (us in a replayed graph, general / chain), 8 heads of 256: 4 rows
+// 2.3 / 3.1, 12 rows 3.0 / 3.2, 16 rows 3.4 / 3.1, 2048 rows 206 / 11.8; 256 heads of 256
+// (4 rounds): 48 rows 8.6 / 10.3, 96 rows 13.3 / 11.0; 256 of 512 (8): 128 rows 16.5 / 19.8,
+// 256 rows 29.2 / 25.0; 512 of 512 (16): 512 rows 59.6 / 64.0, 768 rows 93.9 / 81.6; 1024
+// of 512 (32): 768 rows 138 / 166, 1024 rows 250 / 206.
+inline bool attn_output_chain(uint64_t workgroups, uint32_t seq_len, uint32_t cus) {
+    const uint64_t rounds = (workgroups + cus - 1) / cus;
+    return seq_len >= 1024 || seq_len >= 14 * rounds + 2 * rounds * rounds;
+}
+
 }  // namespace g4

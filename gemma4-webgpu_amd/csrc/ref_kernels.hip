@@ -523,8 +523,8 @@ int g4_attn_output(const float* probs, const uint16_t* v_cache, float* out, g4_a
                     p.num_kv_heads);
     const uint64_t total = (uint64_t)p.num_q_heads * p.head_dim;
     if (total == 0) return G4_OK;
-    if (p.head_dim % 64 == 0 && p.seq_len > 0 && p.seq_len < 0x40000000u && p.num_q_heads <= 65535 &&
-        !(reinterpret_cast<uintptr_t>(v_cache) & 15)) {
+    if (p.head_dim % 64 == 0 && p.seq_len < 0x40000000u && p.num_q_heads <= 65535 &&
+        !(reinterpret_cast<uintptr_t>(v_cache) & 15) && attn_output_chain(total / 64, p.seq_len, device_cus())) {
         G4_LAUNCH(k_attn_output_chain, dim3(p.head_dim / 64, p.num_q_heads), dim3(64 * (kOutMul + 1)), 0,
                   as_stream(stream), probs, v_cache, out, p);
         G4_CHECK_LAUNCH("attnOutput");

@@ -10,11 +10,13 @@
 int main() {
     std::string rule;
     while (std::cin >> rule) {
-        uint32_t a = 0, b = 0;
+        uint32_t a = 0, b = 0, c = 0;
         if (rule == "token_merge_shift" && std::cin >> a)
             printf("%u\n", g4::token_merge_shift(a));
         else if (rule == "softmax_scores_per_thread" && std::cin >> a >> b)
             printf("%u\n", g4::softmax_scores_per_thread(a, b));
+        else if (rule == "attn_output_chain" && std::cin >> a >> b >> c)
+            printf("%d\n", (int)g4::attn_output_chain(a, b, c));
         else
             return fprintf(stderr, "unknown rule %s\n", rule.c_str()), 1;
     }

@@ -6,6 +6,7 @@ import torch
 
 from conftest import announce
 from g4attn import ops
+from helpers import cache_f16
 from oracle import oracle as orc
 from test_gpu_engine_kernels import bits, up
 
@@ -23,3 +24,18 @@ def test_softmax_rule(dev, nh, seq):
     ops.softmax(d, nh, seq)
     torch.cuda.synchronize()
     np.testing.assert_array_equal(bits(d), want.view(np.uint32))
+
+
+@pytest.mark.parametrize("nqh,nkh,hd,seq", [(8, 1, 256, 15), (8, 1, 256, 16), (8, 1, 512, 15), (8, 1, 512, 17), (1, 1, 64, 16),
+                                            (264, 8, 256, 53), (264, 8, 256, 61), (264, 8, 512, 289), (264, 8, 512, 287)])
+def test_attn_output_rule(dev, nqh, nkh, hd, seq):
+    announce(f"attnOutput nqh={nqh} nkh={nkh} hd={hd} seq={seq}")
+    vc = cache_f16(seq + hd, seq, nkh, hd)
+    p = np.random.default_rng(seq).random((nqh, seq), dtype=np.float32) / seq
+    p[:, : seq // 4] = 0.0
+    want = orc.attn_output(p.ravel(), orc.f16_bits_to_f32(vc), nqh, nkh, hd, seq)
+    out = torch.full((nqh * hd + 1,), 7.0, device=dev)
+    ops.attn_output(up(p, dev), up(vc, dev), out, nqh, nkh, hd, seq)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(bits(out)[:-1], want.view(np.uint32))
+    assert float(out[-1]) == 7.0

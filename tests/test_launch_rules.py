@@ -48,3 +48,20 @@ def test_softmax_form_at_the_limits(rule):
         for seq in (1, 512, 513, 4096, 4097, 16384, 16385, 2**32 - 1):
             form = rule("softmax_scores_per_thread", heads, seq)
             assert form in (0, 4, 16) and (not form or 512 < seq <= 1024 * form)
+
+
+@pytest.mark.parametrize("workgroups,seq,chain", [
+    # the general form, measured the faster one
+    (4, 1, 0), (32, 1, 0), (32, 4, 0), (64, 12, 0), (1, 8, 0), (512, 16, 0), (1024, 1, 0), (1024, 48, 0), (2048, 128, 0),
+    (4096, 512, 0), (8192, 768, 0),
+    # the chain form, measured the faster one
+    (1, 16, 1), (32, 16, 1), (64, 64, 1), (64, 2048, 1), (256, 24, 1), (512, 64, 1), (1024, 96, 1), (2048, 256, 1),
+    (4096, 768, 1), (8192, 1024, 1), (8192, 2048, 1)])
+def test_attn_output_form(rule, workgroups, seq, chain):
+    assert rule("attn_output_chain", workgroups, seq, 256) == chain
+
+
+def test_attn_output_form_at_the_limits(rule):
+    for workgroups in (1, 65535 * 8, 2**32 - 1):
+        assert rule("attn_output_chain", workgroups, 0, 256) == 0
+        assert rule("attn_output_chain", workgroups, 2**30 - 1, 1) == 1
