@@ -50,4 +50,10 @@ inline bool attn_output_chain(uint64_t workgroups, uint32_t seq_len, uint32_t cu
     return seq_len >= 1024 || seq_len >= 14 * rounds + 2 * rounds * rounds;
 }
 
+// argmax over few logits takes 256 threads of 4-byte loads: a 1024-thread
+// workgroup's launch and its sixteen candidates cost more than three more loads
+// in turn (us in a replayed graph, 1024 threads / 256: 1 logit 2.5 / 2.2, 255
+// logits 2.7 / 2.2, 768 logits 2.7 / 2.3).
+inline bool argmax_small(uint32_t size) { return size <= 768; }
+
 }  // namespace g4

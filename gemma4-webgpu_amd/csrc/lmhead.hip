@@ -25,6 +25,7 @@
 #include <hip/hip_ext.h>
 
 #include "gemv_core.h"
+#include "launch_rules.h"
 
 namespace g4 {
 
@@ -136,7 +137,7 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
 }
 
 // argmax.wgsl's result by one workgroup (the entry point has no workspace for
-// more). Thread t takes elements VEC t + e + 1024 VEC k: residues mod 256 fixed
+// more). Thread t takes elements VEC t + e + THREADS VEC k: residues mod 256 fixed
 // per (t, e), each kept as its first strict maximum as in the shader; the
 // candidates then meet under the tree's order (lm_candidate). Bound by one CU's
 // load path: kArgmaxBatch 16-byte loads per thread are requested before any is
@@ -147,10 +148,10 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
 constexpr unsigned kArgmaxThreads = 1024;
 constexpr int kArgmaxBatch = 8;
 
-template <int VEC>
-__global__ __launch_bounds__(kArgmaxThreads) void k_argmax(const float* __restrict__ logits, uint32_t* __restrict__ result,
-                                                           uint32_t size) {
-    constexpr uint64_t kStep = (uint64_t)kArgmaxThreads * VEC;
+template <int VEC, unsigned THREADS>
+__global__ __launch_bounds__(THREADS) void k_argmax(const float* __restrict__ logits, uint32_t* __restrict__ result,
+                                                    uint32_t size) {
+    constexpr uint64_t kStep = (uint64_t)THREADS * VEC;
     const unsigned tid = threadIdx.x;
     float best[VEC];
     uint32_t at[VEC];
@@ -193,11 +194,11 @@ __global__ __launch_bounds__(kArgmaxThreads) void k_argmax(const float* __restri
     for (int e = 0; e < VEC; e++) b = max_u64(b, lm_candidate(best[e], at[e]));
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) b = max_u64(b, shfl_xor_u64(b, m));
-    __shared__ uint64_t wbest[kArgmaxThreads / 64];
+    __shared__ uint64_t wbest[THREADS / 64];
     if ((tid & 63) == 0) wbest[tid >> 6] = b;
     __syncthreads();
     if (tid == 0) {
-        for (unsigned w = 1; w < kArgmaxThreads / 64; w++) b = max_u64(b, wbest[w]);
+        for (unsigned w = 1; w < THREADS / 64; w++) b = max_u64(b, wbest[w]);
         result[0] = lm_candidate_row(b);
     }
 }
@@ -400,10 +401,12 @@ int g4_logit_softcap(float* logits, g4_softcap_params p, void* stream) {
 
 int g4_argmax(const float* logits, uint32_t* result, uint32_t size, void* stream) {
     if (!logits || !result) return fail(G4_EINVAL, "argmax: NULL pointer");
-    if (reinterpret_cast<uintptr_t>(logits) & 15)
-        G4_LAUNCH(k_argmax<1>, dim3(1), dim3(kArgmaxThreads), 0, as_stream(stream), logits, result, size);
+    if (argmax_small(size))
+        G4_LAUNCH((k_argmax<1, 256>), dim3(1), dim3(256), 0, as_stream(stream), logits, result, size);
+    else if (reinterpret_cast<uintptr_t>(logits) & 15)
+        G4_LAUNCH((k_argmax<1, kArgmaxThreads>), dim3(1), dim3(kArgmaxThreads), 0, as_stream(stream), logits, result, size);
     else
-        G4_LAUNCH(k_argmax<4>, dim3(1), dim3(kArgmaxThreads), 0, as_stream(stream), logits, result, size);
+        G4_LAUNCH((k_argmax<4, kArgmaxThreads>), dim3(1), dim3(kArgmaxThreads), 0, as_stream(stream), logits, result, size);
     G4_CHECK_LAUNCH("argmax");
     return G4_OK;
 }

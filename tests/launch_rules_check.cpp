@@ -17,6 +17,8 @@ int main() {
             printf("%u\n", g4::softmax_scores_per_thread(a, b));
         else if (rule == "attn_output_chain" && std::cin >> a >> b >> c)
             printf("%d\n", (int)g4::attn_output_chain(a, b, c));
+        else if (rule == "argmax_small" && std::cin >> a)
+            printf("%d\n", (int)g4::argmax_small(a));
         else
             return fprintf(stderr, "unknown rule %s\n", rule.c_str()), 1;
     }

@@ -7,6 +7,7 @@ import torch
 from conftest import announce
 from g4attn import ops
 from helpers import cache_f16
+from oracle import closed_form as cf
 from oracle import oracle as orc
 from test_gpu_engine_kernels import bits, up
 
@@ -39,3 +40,22 @@ def test_attn_output_rule(dev, nqh, nkh, hd, seq):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(bits(out)[:-1], want.view(np.uint32))
     assert float(out[-1]) == 7.0
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("size", [1, 255, 256, 257, 511, 767, 768, 769])
+def test_argmax_rule(dev, size, offset):
+    announce(f"argmax size={size} offset={offset}")
+    rng = np.random.default_rng(size)
+    for trial in range(4):
+        x = rng.integers(-2, 3, size=size).astype(np.float32)  # many ties
+        if trial == 1:
+            x[rng.integers(0, size, size=max(1, size // 3))] = np.nan
+        if trial == 2:
+            x[:] = -np.inf  # no candidate: index 0
+        if trial == 3:
+            x = np.where(x > 0, np.float32(0.0), np.float32(-0.0))  # zeros of both signs compare equal
+        res = torch.full((1,), -1, dtype=torch.int32, device=dev)
+        ops.argmax(up(x, dev, offset), res, size)
+        torch.cuda.synchronize()
+        assert int(res.item()) == orc.argmax(x) == cf.argmax_rule(x), (size, offset, trial)

@@ -65,3 +65,8 @@ def test_attn_output_form_at_the_limits(rule):
     for workgroups in (1, 65535 * 8, 2**32 - 1):
         assert rule("attn_output_chain", workgroups, 0, 256) == 0
         assert rule("attn_output_chain", workgroups, 2**30 - 1, 1) == 1
+
+
+@pytest.mark.parametrize("size,small", [(0, 1), (1, 1), (255, 1), (4096, 0), (262144, 0), (2**32 - 1, 0)])
+def test_argmax_form(rule, size, small):
+    assert rule("argmax_small", size) == small
