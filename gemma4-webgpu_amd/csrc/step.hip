@@ -371,7 +371,11 @@ constexpr uint32_t kStepMagic = 0x67345354u;
 // evaluates and the kernel loads. Planned and run per token (us, host factors / so):
 // 8 sequences of 100 to 1000 rows 17.1 / 13.9, 16 to 3000 rows 23.2 / 17.5, 64 of 100
 // to 600 rows 56.7 / 16.7, 64 of 1K to 32K rows 188.3 / 184.9; 64 at head_dim 512 to
-// 3000 rows 101.4 / 57.9 (the evaluation on the host and 1 KB more to upload per set).
+// 3000 rows 101.4 / 57.9 (the evaluation on the host and 1 KB more to upload per set);
+// at the line, 4 sequences of 50 to 400 rows 17.4 / 13.1, 500 to 3000 rows 17.3 / 14.2, 4K
+// to 16K rows 19.9 / 19.5, at head_dim 512 19.8 / 16.2, 20.4 / 19.3 and 30.3 / 31.0 (long
+// rows hide the host's work). The evaluation itself costs a step 0.3 to 0.5 us, at head_dim
+// 512 1.0 to 1.3, which a plan that is run again without an advance pays each time.
 constexpr uint32_t kStepRopeEvalSets = 4;
 
 struct StepPlanRep {
