@@ -1129,10 +1129,10 @@ int build(const g4_prefill_entry* ents, uint32_t n, uint32_t nqh, uint32_t nkh, 
         // 168 us against 177 us at 1536 and 183 us at 3840. At least 256 keys, or 160 where parts of
         // 256 would leave two thirds of the CUs idle and a merge is due anyway (a longer tile than
         // 256): an item's time is its fixed cost and ~1 us per 32 keys. Measured, 256 / 160 (us, kept
-        // plans): 30 tokens after 2000 cached 26.7 / 25.1, 80 after 800 27.0 / 25.6, 5 after 3000 on one
-        // layer 23.8 / 21.6; head_dim 512: 8 after 1500 35.4 / 30.2, 80 after 500 35.5 / 32.5. With more
-        // items the longer merges cost more: head_dim 512, 500 tokens 34.9 / 35.8; 143 tokens alone
-        // (no merge at 256) 20.2, 22.9 in parts of 128.
+        // plans with their prep): 30 tokens after 2000 cached 27.1 / 26.3, 80 after 800 27.3 / 26.1, 5 after
+        // 3000 on one layer 24.9 / 22.3; head_dim 512: 8 after 1500 35.5 / 30.5, 80 after 500 35.5 / 32.9.
+        // With more items the longer merges cost more: head_dim 512, 500 tokens 34.9 / 35.8; 143 tokens
+        // alone (no merge at 256) 20.2, 22.9 in parts of 128.
         uint64_t w = 0, long_items = 0;  // long_items: with parts of kPfPartKeys
         uint32_t longest = 0;
         for (uint32_t i = 0; i < n; i++) {

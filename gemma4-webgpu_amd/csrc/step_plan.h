@@ -502,9 +502,9 @@ inline int plan_step(const g4_step_entry* entries, uint32_t n_entries, uint32_t 
     // different queries) go to one XCD, whose L2 then reads those rows once for
     // all of them; the parts go to the XCD with the most workgroups left (groups
     // first), which spreads the distinct rows evenly too. Measured on a token of
-    // E2B's real shapes (us, two states in turn): position 32768 80.9 entry by entry
-    // with streaming loads, 64.1 so with ordinary ones (73.7 so with streaming ones);
-    // 16384 56.0 / 37.1, 8192 37.3 / 27.9, 2048 23.0 / 19.1. With the groups' parts on
+    // E2B's real shapes (us, two states in turn): position 32768 81.8 entry by entry
+    // with streaming loads, 63.2 so with ordinary ones (72.0 so with streaming ones);
+    // 16384 56.0 / 36.4, 8192 37.0 / 26.5, 2048 22.9 / 18.9. With the groups' parts on
     // consecutive XCDs, not spread, 32768 took 69.0: the entries without a group then
     // sat on two XCDs, whose share of the memory bandwidth bounded the launch.
     uint64_t next[kXcds], left[kXcds];  // an XCD's next workgroup, and how many it has left

@@ -42,7 +42,7 @@ struct StepEntryDev {
     uint32_t key_end;   // one past the last attended row; the current row is key_end - 1
     uint32_t n_parts;   // workgroups on this entry
     uint32_t position;  // RoPE position
-    uint32_t flags;     // kStoreKv | kRowCached | kApplyDivisor | kRopeEval | kQReady | kQReady
+    uint32_t flags;     // kStoreKv | kRowCached | kApplyDivisor | kRopeEval | kQReady
     float theta;
     uint32_t window;    // sliding window (0 = full): rows [key_end - window, key_end) when key_end > window
     float qscale;       // attention scale * log2(e)

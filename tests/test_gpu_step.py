@@ -278,7 +278,7 @@ HD512 = [  # (seq, window, theta, divisor): E2B global layers have head_dim 512
 
 @pytest.mark.parametrize("seq,win,theta,div", HD512)
 def test_step_head_dim_512(dev, seq, win, theta, div):
-    """head_dim 512 (one 4-wave workgroup per CU): the stored rows bit-identical, attnOut within 2e-3, with and
+    """head_dim 512 (one 8-wave workgroup per CU): the stored rows bit-identical, attnOut within 2e-3, with and
     without the host RoPE table (same bits)."""
     announce(f"attnStep hd=512 seq={seq} win={win}")
     L = Layer(dev, 600 + seq, seq, win, theta, div, hd=512)
